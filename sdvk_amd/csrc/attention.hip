@@ -20,10 +20,9 @@
 //   * O^T = V^T P^T on the same MFMA: P stays in registers (the S^T output
 //     layout is, key for key, the B-operand layout the PV product needs); V is
 //     stored in LDS grouped by the PV step that consumes each key, so each A
-//     fragment is one 16-byte read; the row sums of P come from the same MFMA
-//     (an all-ones A operand) in the fp32-input kernel, and from v_dot2_f32_f16
-//     on the fp16 P values in the fp16 kernel (VALU instead of a fifth of its
-//     MFMAs);
+//     fragment is one 16-byte read; the row sums of P come from v_dot2_f32_f16 on
+//     the fp16 P values (VALU instead of a fifth of the MFMAs), or from the same
+//     MFMA (an all-ones A operand) in the element-wise kernel;
 //   * fp32 inputs (the reference layout) are carried as fp16 hi + lo pairs
 //     (x = hi + lo to 2^-22): S = K_hi Q_hi + K_lo Q_hi + K_hi Q_lo and
 //     O = V_hi P + V_lo P, so only P is rounded to fp16. fp16 inputs take one
@@ -69,36 +68,16 @@ struct AttnArgs {
     float* part;
 };
 
-// 8 consecutive elements as fp16 (hi); for fp32 sources also the residual
-// lo = fp16(x - hi), so that hi + lo carries x to 2^-22 relative.
+// 8 consecutive elements as fp16 (hi), those at or past `valid` zero; for fp32
+// sources also the residual lo = fp16(x - hi), so that hi + lo carries x to
+// 2^-22 relative.
 template <typename T>
-__device__ __forceinline__ void load8(const T* p, bool vec, int valid, half8& hi, half8& lo) {
-    if constexpr (sizeof(T) == 2) {
-        if (vec) {
-            hi = *reinterpret_cast<const half8*>(p);
-        } else {
+__device__ __forceinline__ void load8(const T* p, int valid, half8& hi, half8& lo) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) hi[i] = i < valid ? p[i] : static_cast<_Float16>(0.0f);
-        }
-    } else {
-        float x[8];
-        if (vec) {
-            floatx4 a = reinterpret_cast<const floatx4*>(p)[0];
-            floatx4 b = reinterpret_cast<const floatx4*>(p)[1];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                x[i] = a[i];
-                x[4 + i] = b[i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) x[i] = i < valid ? p[i] : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            hi[i] = static_cast<_Float16>(x[i]);
-            lo[i] = static_cast<_Float16>(x[i] - static_cast<float>(hi[i]));
-        }
+    for (int i = 0; i < 8; ++i) {
+        const T x = i < valid ? p[i] : static_cast<T>(0.0f);
+        hi[i] = static_cast<_Float16>(x);
+        if constexpr (sizeof(T) == 4) lo[i] = static_cast<_Float16>(x - static_cast<float>(hi[i]));
     }
 }
 
@@ -106,27 +85,12 @@ __device__ __forceinline__ half8 zero8() { return half8{0, 0, 0, 0, 0, 0, 0, 0};
 
 // 4 consecutive elements as fp16 (hi) and, for fp32 sources, the residual lo.
 template <typename T>
-__device__ __forceinline__ void load4(const T* p, bool vec, int valid, half4& hi, half4& lo) {
-    if constexpr (sizeof(T) == 2) {
-        if (vec) {
-            hi = *reinterpret_cast<const half4*>(p);
-        } else {
+__device__ __forceinline__ void load4(const T* p, int valid, half4& hi, half4& lo) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) hi[i] = i < valid ? p[i] : static_cast<_Float16>(0.0f);
-        }
-    } else {
-        floatx4 x;
-        if (vec) {
-            x = *reinterpret_cast<const floatx4*>(p);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[i] = i < valid ? p[i] : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            hi[i] = static_cast<_Float16>(x[i]);
-            lo[i] = static_cast<_Float16>(x[i] - static_cast<float>(hi[i]));
-        }
+    for (int i = 0; i < 4; ++i) {
+        const T x = i < valid ? p[i] : static_cast<T>(0.0f);
+        hi[i] = static_cast<_Float16>(x);
+        if constexpr (sizeof(T) == 4) lo[i] = static_cast<_Float16>(x - static_cast<float>(hi[i]));
     }
 }
 
@@ -217,8 +181,12 @@ constexpr float kLazy = 8.0f;
 // P <= 2^kLazy.
 constexpr float kLazySum = 256.0f;
 
+// Tensors whose rows are not 16-byte aligned, or with a head dim that is not a
+// multiple of 8: element-wise loads and stores (VEC = false, the only build: the
+// others take the pipelined kernels below).
 template <typename TI, typename TO, bool VEC>
 __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
+    static_assert(!VEC, "16-byte aligned tensors take the pipelined kernels");
     constexpr bool kSplit = sizeof(TI) == 4;  // fp32 inputs: hi + lo planes
     constexpr int NP = kSplit ? 2 : 1;
     __shared__ __attribute__((aligned(16))) _Float16 Ks[2][NP][kBKV * kKld];
@@ -256,7 +224,7 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
         const int valid = hd - d0;
         qf[s] = zero8();
         qlo[s] = zero8();
-        if (qi < a.Tq && valid > 0) load8(Qp + static_cast<uint64_t>(qi) * a.ldq + d0, VEC, valid, qf[s], qlo[s]);
+        if (qi < a.Tq && valid > 0) load8(Qp + static_cast<uint64_t>(qi) * a.ldq + d0, valid, qf[s], qlo[s]);
     }
 
     // Staging. K: chunks of 8 d (thread handles chunks tid and tid + 256: key =
@@ -269,75 +237,26 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
     half8 kreg[2][NP];
     half4 vreg[4][NP];
     const int vkg = tid & 15, vd0 = (tid >> 4) * 4;
-    // Vector path: K/V rows through buffer resources whose base advances with
-    // the tile (scalar work only) and whose size ends at key L-1, so rows past
-    // the valid keys read as zeros (hardware range check) with no lane guards.
-    // Chunks at d >= hd take an offset past every record (the load returns
-    // zeros) instead of reading the neighbouring head's columns.
-    const bool kin = (tid & 7) * 8 < hd;
-    const uint32_t k_off0 = kin ? ((tid >> 3) * static_cast<uint32_t>(a.ldk) + (tid & 7) * 8) * sizeof(TI) : kOob;
-    const uint32_t k_off1 = kin ? k_off0 + 32u * static_cast<uint32_t>(a.ldk) * sizeof(TI) : kOob;
-    const uint32_t v_off = vd0 < hd ? (vkg * 4 * static_cast<uint32_t>(a.ldv) + vd0) * sizeof(TI) : kOob;
-    const uint32_t v_row = static_cast<uint32_t>(a.ldv) * sizeof(TI);
     auto load_tile = [&](uint32_t kv0) {
-        if constexpr (VEC) {
-            const uint32_t kbytes = tile_bytes(kv0, L, a.ldk, a.hd, sizeof(TI));
-            const uint32_t vbytes = tile_bytes(kv0, L, a.ldv, a.hd, sizeof(TI));
-            const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<TI*>(Kp + static_cast<uint64_t>(kv0) * a.ldk), 0, static_cast<int>(kbytes), 0x00020000);
-            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-                const_cast<TI*>(Vp + static_cast<uint64_t>(kv0) * a.ldv), 0, static_cast<int>(vbytes), 0x00020000);
-            if constexpr (sizeof(TI) == 2) {
-                kreg[0][0] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rk, k_off0, 0, 0));
-                kreg[1][0] = __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(rk, k_off1, 0, 0));
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    vreg[i][0] = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(rv, v_off + i * v_row, 0, 0));
-            } else {
+        for (int i = 0; i < 2; ++i) {
+            const int c = tid + i * kThreads;
+            const uint32_t key = kv0 + (c >> 3);
+            const int d0 = (c & 7) * 8;
+            const int valid = hd - d0;
+            half8 klo = zero8();
+            kreg[i][0] = zero8();
+            if (key < L && valid > 0) load8(Kp + static_cast<uint64_t>(key) * a.ldk + d0, valid, kreg[i][0], klo);
+            if constexpr (kSplit) kreg[i][NP - 1] = klo;
+        }
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const uint32_t off = i ? k_off1 : k_off0;
-                    const floatx4 x0 = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 0));
-                    const floatx4 x1 = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16, 0, 0));
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        kreg[i][0][e] = static_cast<_Float16>(x0[e]);
-                        kreg[i][0][4 + e] = static_cast<_Float16>(x1[e]);
-                        kreg[i][NP - 1][e] = static_cast<_Float16>(x0[e] - static_cast<float>(kreg[i][0][e]));
-                        kreg[i][NP - 1][4 + e] = static_cast<_Float16>(x1[e] - static_cast<float>(kreg[i][0][4 + e]));
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const floatx4 x = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rv, v_off + i * v_row, 0, 0));
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        vreg[i][0][e] = static_cast<_Float16>(x[e]);
-                        vreg[i][NP - 1][e] = static_cast<_Float16>(x[e] - static_cast<float>(vreg[i][0][e]));
-                    }
-                }
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int c = tid + i * kThreads;
-                const uint32_t key = kv0 + (c >> 3);
-                const int d0 = (c & 7) * 8;
-                const int valid = hd - d0;
-                half8 klo = zero8();
-                kreg[i][0] = zero8();
-                if (key < L && valid > 0) load8(Kp + static_cast<uint64_t>(key) * a.ldk + d0, VEC, valid, kreg[i][0], klo);
-                if constexpr (kSplit) kreg[i][NP - 1] = klo;
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t key = kv0 + vkg * 4 + i;
-                const int valid = hd - vd0;
-                half4 vlo = half4{0, 0, 0, 0};
-                vreg[i][0] = half4{0, 0, 0, 0};
-                if (key < L && valid > 0) load4(Vp + static_cast<uint64_t>(key) * a.ldv + vd0, VEC, valid, vreg[i][0], vlo);
-                if constexpr (kSplit) vreg[i][NP - 1] = vlo;
-            }
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t key = kv0 + vkg * 4 + i;
+            const int valid = hd - vd0;
+            half4 vlo = half4{0, 0, 0, 0};
+            vreg[i][0] = half4{0, 0, 0, 0};
+            if (key < L && valid > 0) load4(Vp + static_cast<uint64_t>(key) * a.ldv + vd0, valid, vreg[i][0], vlo);
+            if constexpr (kSplit) vreg[i][NP - 1] = vlo;
         }
     };
     auto store_tile = [&](int st) {
@@ -487,15 +406,456 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
 
     const float lt = o[2][0];
     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
-    constexpr int kWaveBytes = 32 * 64 * static_cast<int>(sizeof(TO));
-    if constexpr (VEC && static_cast<int>(sizeof(Ks)) >= (kThreads / 64) * kWaveBytes) {
-        if (a.ostage) {  // through LDS (the K stages, free after every wave's last tile)
-            __syncthreads();
-            const int nrows = qwave >= a.Tq ? 0 : static_cast<int>(min(a.Tq - qwave, 32u));
-            TO* Ob = static_cast<TO*>(a.o) + b * a.so + static_cast<uint64_t>(qwave) * a.ldo + static_cast<uint64_t>(h) * a.hd;
-            store_o_rows<TO>(o, inv, reinterpret_cast<char*>(&Ks[0][0][0]) + wave * kWaveBytes, Ob, nrows, hd, a.ldo, lane);
-            return;
+    if (qi >= a.Tq) return;
+    TO* Op = static_cast<TO*>(a.o) + b * a.so + static_cast<uint64_t>(qi) * a.ldo + static_cast<uint64_t>(h) * a.hd;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int run = 0; run < 4; ++run) {
+            const int d0 = 32 * u + 8 * run + 4 * g;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (d0 + e < hd) Op[d0 + e] = static_cast<TO>(o[u][4 * run + e] * inv);
         }
+}
+
+
+// RESID: which tiles add P's fp16 residual as a second PV product, at compile
+// time (a runtime test of the flag inside the loop cost non-causal launches
+// 2.4%): kResidNone; kResidDiagonal, a causal launch's diagonal tiles;
+// kResidAll, every tile (MI_ATTN_PREC_SPLIT).
+constexpr int kResidNone = 0, kResidDiagonal = 1, kResidAll = 2;
+
+// ---- fp32 inputs: software-pipelined kernel ---------------------------------
+//
+// attn_kernel's arithmetic for fp32 tensors (Q, K, V as fp16 hi + lo pairs, three
+// MFMAs per score fragment), arranged so that the vector work fits under the
+// MFMAs of the same wave:
+//
+//   * keys are taken 32 at a time (two sub-tiles per staged 64-key tile). Phase A
+//     issues the score MFMAs of the next sub-tile between the exponentials and
+//     fp16 packing of this one; phase B issues this sub-tile's PV MFMAs between
+//     the conversion and LDS stores of the next tile;
+//   * the running max enters as the score MFMA's initial accumulator (-m, in raw
+//     score units, one register block that changes only when m does), so an
+//     exponential costs one multiply by scale * log2 e and the exp itself;
+//   * as in the fp16 kernel no row max is taken per tile: the sum of a sub-tile's P
+//     bounds each of them, and a sum over 2^8 (rare) sends the wave through a
+//     rescale;
+//   * P V = V_hi P_hi + V_lo P_hi (+ V_hi P_lo where P's residual counts, RESID as
+//     in the fp16 kernel): V_lo P_lo is below 2^-22 of a product and left out. The
+//     row sums are VALU adds, not an all-ones MFMA operand;
+//   * hi = fp16(x) and lo = fp16(x - hi) take 1.5 instructions per element (packed
+//     conversion, then a mixed-precision fma that rounds straight to fp16).
+//
+// KG = 2: eight waves, two groups of four over the same 128 queries; group g
+// takes key tiles g, g + 2, ... through LDS stages of its own and the groups'
+// partial results are added at the end through LDS (group 0 + group 1, a fixed
+// order). It is taken where the grid has at most one workgroup per CU, which
+// would leave one wave on each SIMD.
+//
+// One barrier per tile: a trip's PV phases store the next tile's V and the K of
+// the tile after it, each into a half stage whose last readers passed the trip's
+// barrier. LDS: two stages of 36 KB per group (two workgroups of KG = 1 or one of
+// KG = 2 per CU, two waves per SIMD either way).
+//
+// What bounds it: MFMA and VALU issue, close together. Per wave, 64 keys and 32
+// queries: 24 score + 16 PV MFMAs (24 with P's residual) of 34 cycles, and 32
+// multiplies, 32 exponentials (8.5 cycles each), 32 packed conversions and 32 or 64
+// mixed fmas (9 cycles each) on the VALU. Measured on MI355X against the unpipelined
+// kernel it replaces, us: mi_fused_attention 1 x 10 x 2304^2 77.3 -> 48.7 (280
+// TFLOP/s), 1 x 10 x 4096^2 219 -> 165, 2 x 10 x 4096^2 with fp16 P 290 -> 234, cross
+// 2 x 10 x 4096 x 77 22.8 -> 20.0; error against 64 bits 6.8e-7 -> 4.7e-7 of the
+// result's norm (2304 keys, N(0, 1) data).
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+// Two values as fp16 (RNE) in one packed conversion.
+__device__ __forceinline__ half2 pack2(float x, float y) { return __builtin_convertvector(floatx2{x, y}, half2); }
+// fp16(x - hi): neg1 holds -1 in a register the compiler cannot see through, so
+// the subtraction stays a fma that rounds straight to fp16 (v_fma_mixlo/hi_f16).
+__device__ __forceinline__ half2 residual2(half2 hi, float x, float y, float neg1) {
+    return half2{static_cast<_Float16>(__builtin_fmaf(static_cast<float>(hi[0]), neg1, x)),
+                 static_cast<_Float16>(__builtin_fmaf(static_cast<float>(hi[1]), neg1, y))};
+}
+
+constexpr int kFLd = 72;                    // halves per staged row: 64 + 16-byte pad
+constexpr int kFPlane = kBKV * kFLd;        // halves of one staged plane (K or V, hi or lo)
+constexpr int kFStage = 4 * kFPlane;        // K hi, K lo, V hi, V lo
+constexpr int kFQRow = 68;                  // floats per staged Q row: 64 + 16-byte pad
+
+template <typename TO, int RESID, int KG>
+__global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint32_t qtiles) {
+    __shared__ __attribute__((aligned(16))) _Float16 smem[KG * 2 * kFStage];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, tg = tid & 255;
+    const int wave = __builtin_amdgcn_readfirstlane((tid >> 6) & 3);  // wave-uniform: scalar mask tests
+    const int grp = KG == 2 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;
+    const int l32 = lane & 31, g = lane >> 5;
+    _Float16* const stage0 = smem + grp * 2 * kFStage;
+
+    const uint32_t blk = xcd_swizzle(blockIdx.x, gridDim.x);
+    const uint32_t qt = blk % qtiles, bh = blk / qtiles;
+    const uint32_t h = bh % a.heads, b = bh / a.heads;
+    const uint32_t qcta = qt * kBQ, qwave = qcta + wave * 32, qi = qwave + l32;
+    const int hd = static_cast<int>(a.hd);
+
+    uint32_t L = a.Tk;
+    if (a.kv_len) {
+        int32_t l = a.kv_len[b];
+        L = l < 0 ? 0u : (static_cast<uint32_t>(l) < a.Tk ? static_cast<uint32_t>(l) : a.Tk);
+    }
+    uint32_t kend = L;
+    if (a.causal) kend = min(kend, qcta + kBQ);
+    // sub-tiles that end at or before kfull need no mask for any query of this wave
+    uint32_t kfull = L / 32 * 32;
+    if (a.causal) kfull = min(kfull, (qwave + 1) / 32 * 32);
+    const uint32_t ntiles = (kend + kBKV - 1) / kBKV;
+    // tiles of this group: grp, grp + KG, ...; every group runs n trips (the
+    // barriers are the workgroup's), a trip past ntiles finds every key masked
+    const uint32_t n = (ntiles + KG - 1) / KG;
+
+    const float* Qp = static_cast<const float*>(a.q) + b * a.sq + static_cast<uint64_t>(h) * a.hd;
+    const float* Kp = static_cast<const float*>(a.k) + b * a.sk + static_cast<uint64_t>(h) * a.hd;
+    const float* Vp = static_cast<const float*>(a.v) + b * a.sv + static_cast<uint64_t>(h) * a.hd;
+
+    // K: 16-byte unit (row tg / 16 + 16 i, columns 4 (tg % 16)): a wave's load
+    // covers four whole 256-byte rows. V: rows 4 kg + i at columns 4 (lane % 16),
+    // four whole rows again; the 4 x 4 block is transposed by the packing.
+    const int krow = tg >> 4, kcol = (tg & 15) * 4;
+    const int vn = lane & 15, vp = lane >> 4;
+    const int kg4 = 4 * wave + ((vp & 1) << 1 | vp >> 1);  // lanes 0-31 write both halves of a 16-byte unit
+    const uint32_t k_ld4 = static_cast<uint32_t>(a.ldk) * 4, v_ld4 = static_cast<uint32_t>(a.ldv) * 4;
+    const uint32_t k_off = kcol < hd ? krow * k_ld4 + kcol * 4 : kOob;
+    const uint32_t v_off = 4 * vn < hd ? 4 * kg4 * v_ld4 + vn * 16 : kOob;
+    float neg1 = -1.0f;
+    asm volatile("" : "+v"(neg1));
+    floatx4 kraw[4], vraw[4];
+    // rows past the keys read as zeros (the resource ends at key L - 1)
+    auto load_k = [&](uint32_t trip) {
+        const uint32_t kv0 = (trip * KG + grp) * kBKV;
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(Kp + static_cast<uint64_t>(min(kv0, L)) * a.ldk), 0,
+            static_cast<int>(tile_bytes(kv0, L, a.ldk, a.hd, 4)), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            kraw[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, k_off + i * 16u * k_ld4, 0, 0));
+    };
+    auto load_v = [&](uint32_t trip) {
+        const uint32_t kv0 = (trip * KG + grp) * kBKV;
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float*>(Vp + static_cast<uint64_t>(min(kv0, L)) * a.ldv), 0,
+            static_cast<int>(tile_bytes(kv0, L, a.ldv, a.hd, 4)), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            vraw[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, v_off + i * v_ld4, 0, 0));
+    };
+    // Staged K: row-major, row stride kFLd. Staged V: row d holds the 64 keys as
+    // eight 16-byte units, unit G = (t, sp, g) the keys that lane half g of PV
+    // step (t, sp) consumes (key 32t + 16sp + 8j + 4g + i in slot 4j + i), at
+    // place G ^ ((d / 16) % 4): the 8-byte stores of 32 lanes then cover all 64
+    // banks once, and a fragment is one 16-byte read.
+    const int vG = (kg4 >> 3) * 4 + ((kg4 >> 2) & 1) * 2 + (kg4 & 1);
+    const int v_st = 4 * vn * kFLd + (vG ^ ((vn >> 2) & 3)) * 8 + ((kg4 >> 1) & 1) * 4;
+    const int k_st = krow * kFLd + kcol;
+    // unit 0..3: the thread's K units; 4..7: its V columns (4 keys each)
+    auto store_unit = [&](int st, int i) {
+        _Float16* S = stage0 + st * kFStage + (i < 4 ? k_st + i * 16 * kFLd : 2 * kFPlane + v_st + (i - 4) * kFLd);
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = i < 4 ? kraw[i & 3][e] : vraw[e][i & 3];
+        const half2 h0 = pack2(x[0], x[1]), h1 = pack2(x[2], x[3]);
+        const half2 l0 = residual2(h0, x[0], x[1], neg1), l1 = residual2(h1, x[2], x[3], neg1);
+        *reinterpret_cast<half4*>(S) = half4{h0[0], h0[1], h1[0], h1[1]};
+        *reinterpret_cast<half4*>(S + kFPlane) = half4{l0[0], l0[1], l1[0], l1[1]};
+    };
+
+    half8 qh[4], ql[4];
+    floatx16 o[2], mneg;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[0][r] = o[1][r] = mneg[r] = 0.0f;
+    float lsum = 0.0f, m = 0.0f;
+    const float c = fabsf(a.c);  // a negative scale is taken into Q
+
+    const int k_rd = l32 * kFLd + 8 * g, v_rd = l32 * kFLd + (g ^ (l32 >> 4)) * 8;
+    // K fragments of sub-tile t's k-slice s4 (16 of the 64 columns)
+    half8 kh[4], kl[4];
+    auto read_k = [&](int st, int t, int s4) {
+        const _Float16* S = stage0 + st * kFStage + k_rd + 32 * t * kFLd + 16 * s4;
+        kh[s4] = *reinterpret_cast<const half8*>(S);
+        kl[s4] = *reinterpret_cast<const half8*>(S + kFPlane);
+    };
+    // V^T fragments of PV step (t, sp), columns 32u .. 32u + 31
+    half8 vh[2][2], vl[2][2];
+    auto read_v = [&](int st, int t, int sp) {
+        const _Float16* S = stage0 + st * kFStage + 2 * kFPlane + v_rd;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            // row 32u + l32, unit (4t + 2sp + g) ^ (2u + l32 / 16) = 4t + 2(sp ^ u) + (g ^ l32 / 16)
+            const int off = 32 * u * kFLd + 32 * t + 16 * (sp ^ u);
+            vh[sp][u] = *reinterpret_cast<const half8*>(S + off);
+            vl[sp][u] = *reinterpret_cast<const half8*>(S + kFPlane + off);
+        }
+    };
+    auto mask = [&](floatx16& s, uint32_t k0) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t key = k0 + 8 * (r >> 2) + 4 * g + (r & 3);
+            if (key >= L || (a.causal && key > qi)) s[r] = -INFINITY;
+        }
+    };
+    auto lane_max = [&](const floatx16& s) {
+        float mx = s[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+        return fmaxf(mx, __shfl_xor(mx, 32));  // the partner lane holds the query's other 16 keys
+    };
+    // p: P of a sub-tile in fp32, ph its fp16 rounding (pair i = scores 2i, 2i + 1);
+    // ts: the lane's sum of ph (summing what was packed also keeps the packing
+    // ahead of settle's branch, under the MFMAs). pl = fp16(p - ph), added to the
+    // row sum directly.
+    floatx16 p;
+    half2 ph[8], pl[8];
+    float ts;
+    const half2 one2 = {1, 1};
+    auto exps = [&](const floatx16& s, int i) {
+        p[2 * i] = __builtin_amdgcn_exp2f(s[2 * i] * c);
+        p[2 * i + 1] = __builtin_amdgcn_exp2f(s[2 * i + 1] * c);
+    };
+    auto soft = [&](const floatx16& s, int i) {  // the next pair's exponentials, then pack pair i
+        if (i < 7) exps(s, i + 1);
+        ph[i] = pack2(p[2 * i], p[2 * i + 1]);
+        ts = __builtin_amdgcn_fdot2(ph[i], one2, ts, false);
+    };
+    auto residual = [&](int i) {  // pairs i, i + 1
+        pl[i] = residual2(ph[i], p[2 * i], p[2 * i + 1], neg1);
+        pl[i + 1] = residual2(ph[i + 1], p[2 * i + 2], p[2 * i + 3], neg1);
+        lsum = __builtin_amdgcn_fdot2(pl[i], one2, lsum, false);
+        lsum = __builtin_amdgcn_fdot2(pl[i + 1], one2, lsum, false);
+    };
+    auto frag = [](const half2 (&x)[8], int sp) {
+        const half2* y = x + 4 * sp;
+        return half8{y[0][0], y[0][1], y[1][0], y[1][1], y[2][0], y[2][1], y[3][0], y[3][1]};
+    };
+    // Adds the sub-tile's sum after the lazy-rescale test; next: the scores of
+    // the following sub-tile, already taken against the old m.
+    auto settle = [&](floatx16& s, floatx16& next) {
+        if (__any(ts > kLazySum)) {
+            const float d = fmaxf(lane_max(s), 0.0f);
+            const float alpha = __builtin_amdgcn_exp2f(-d * c);
+            m += d;
+            lsum *= alpha;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                o[0][r] *= alpha;
+                o[1][r] *= alpha;
+                mneg[r] = -m;
+                s[r] -= d;
+                next[r] -= d;
+            }
+            ts = 0.0f;
+            exps(s, 0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) soft(s, i);
+        }
+        lsum += ts;
+    };
+    // Phase A: next = scores of sub-tile (st, t) against m (12 MFMAs in a chain),
+    // P of s between them; the first V fragments of the PV phase (vst, vt) that
+    // follows are read at its end. The scheduler's barriers hold each piece of
+    // vector work behind its MFMA (left alone the compiler issues the MFMAs in a
+    // burst).
+    auto phase_a = [&](const floatx16& s, floatx16& next, int st, int t, auto VNEXT, int vst, int vt) {
+        ts = 0.0f;
+        exps(s, 0);
+        next = mneg;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4) {
+            if (s4 < 2) read_k(st, t, s4 + 2);
+            if (decltype(VNEXT)::value && s4 == 3) read_v(vst, vt, 0);
+            next = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[s4], qh[s4], next, 0, 0, 0);
+            soft(s, 2 * s4);
+            __builtin_amdgcn_sched_barrier(0);
+            next = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[s4], ql[s4], next, 0, 0, 0);
+            soft(s, 2 * s4 + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            next = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[s4], qh[s4], next, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // Phase B: PV of sub-tile (st, t); between its MFMAs the conversion of four
+    // units (V of the next tile in the first phase of a trip, K of the tile after
+    // it in the second) into stage wst, and P's residual; at its end the first K
+    // fragments of the score phase (kst, kt) that follows.
+    auto phase_b = [&](auto VREAD, int st, int t, int wst, int unit0, int kst, int kt) {
+        constexpr bool kRes = RESID != kResidNone;
+        if (!decltype(VREAD)::value) read_v(st, t, 0);
+        read_v(st, t, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (kRes) residual(0);
+        else store_unit(wst, unit0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int sp = i >> 2, u = i & 1;
+            const half8 v = i & 2 ? vl[sp][u] : vh[sp][u];
+            o[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, frag(ph, sp), o[u], 0, 0, 0);
+            if constexpr (kRes) {
+                if (!(i & 1) && i < 6) residual(i + 2);
+                else if (i == 5 || i == 7) store_unit(wst, unit0 + (i >> 1) - 2);
+            } else {
+                if (!(i & 1) && i < 6) store_unit(wst, unit0 + 1 + (i >> 1));
+                if (i == 5) read_k(kst, kt, 0);
+                if (i == 7) read_k(kst, kt, 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (kRes) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                o[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i >> 1][i & 1], frag(pl, i >> 1), o[i & 1], 0, 0, 0);
+                if (i < 2) store_unit(wst, unit0 + 2 + i);
+                if (i >= 2) read_k(kst, kt, i - 2);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+
+    if (n > 0) {
+        // Q rows of this wave (whole 256-byte rows per load), through the second
+        // stage's space; then tile 0 into the first stage
+        {
+            const uint32_t nq = qwave < a.Tq ? min(a.Tq - qwave, 32u) : 0u;
+            const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<float*>(Qp + static_cast<uint64_t>(nq ? qwave : 0u) * a.ldq), 0,
+                nq ? static_cast<int>(((nq - 1) * a.ldq + a.hd) * 4) : 0, 0x00020000);
+            floatx4 qraw[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t row = 4 * i + (lane >> 4);
+                qraw[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                    rq, 4 * vn < hd ? row * static_cast<uint32_t>(a.ldq) * 4u + vn * 16u : kOob, 0, 0));
+            }
+            load_k(0);
+            load_v(0);
+            float* Q = reinterpret_cast<float*>(stage0 + kFStage) + wave * 32 * kFQRow;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                *reinterpret_cast<floatx4*>(Q + (4 * i + (lane >> 4)) * kFQRow + 4 * vn) = qraw[i];
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int s4 = 0; s4 < 4; ++s4)
+#pragma unroll
+                for (int e4 = 0; e4 < 2; ++e4) {
+                    const floatx4 x = *reinterpret_cast<const floatx4*>(Q + l32 * kFQRow + 16 * s4 + 8 * g + 4 * e4);
+#pragma unroll
+                    for (int e = 0; e < 4; e += 2) {
+                        const float v0 = a.c < 0.0f ? -x[e] : x[e], v1 = a.c < 0.0f ? -x[e + 1] : x[e + 1];
+                        const half2 hi = pack2(v0, v1), lo = residual2(hi, v0, v1, neg1);
+                        qh[s4][4 * e4 + e] = hi[0];
+                        qh[s4][4 * e4 + e + 1] = hi[1];
+                        ql[s4][4 * e4 + e] = lo[0];
+                        ql[s4][4 * e4 + e + 1] = lo[1];
+                    }
+                }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) store_unit(0, i);
+            load_k(min(1u, n - 1));
+        }
+        __syncthreads();  // every wave has read its Q rows out of the second stage
+#pragma unroll
+        for (int i = 0; i < 4; ++i) store_unit(1, i);
+        load_v(min(1u, n - 1));  // V before K, as in the loop (loads retire in issue order)
+        load_k(min(2u, n - 1));
+        floatx16 s0 = mneg, s1;
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4) {
+            read_k(0, 0, s4);
+            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[s4], qh[s4], s0, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[s4], ql[s4], s0, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[s4], qh[s4], s0, 0, 0, 0);
+        }
+        if (grp * kBKV + 32 > kfull) mask(s0, grp * kBKV);
+        // the first sub-tile's max (a group whose first sub-tile is masked for a
+        // query has no key of that query at all: its keys only ascend)
+        const float mx0 = lane_max(s0);
+        m = mx0 == -INFINITY ? 0.0f : mx0;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            mneg[r] = -m;
+            s0[r] -= m;
+        }
+        read_k(0, 1, 0);
+        read_k(0, 1, 1);
+        // At the top of trip j: K tiles j and j + 1 and V tile j staged (or being
+        // stored, before the first barrier), K tile j + 2 and V tile j + 1 on their
+        // way into registers; s0 holds the scores of sub-tile 0. Past the last tile
+        // the loads repeat it: scores nobody reads.
+        for (uint32_t j = 0; j < n; ++j) {
+            const int st = j & 1;
+            const uint32_t kv0 = (j * KG + grp) * kBKV;
+            phase_a(s0, s1, st, 1, std::false_type{}, st, 0);
+            settle(s0, s1);
+            if (kv0 + 64 > kfull) mask(s1, kv0 + 32);
+            // tile j's V and tile j + 1's K are whole; every wave is done with tile
+            // j's K and tile j - 1's V
+            __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
+            phase_b(std::false_type{}, st, 0, st ^ 1, 4, st ^ 1, 0);
+            load_v(min(j + 2, n - 1));
+            __builtin_amdgcn_sched_barrier(0);
+            phase_a(s1, s0, st ^ 1, 0, std::true_type{}, st, 1);
+            settle(s1, s0);
+            if (kv0 + KG * kBKV + 32 > kfull) mask(s0, kv0 + KG * kBKV);
+            __builtin_amdgcn_sched_barrier(0);
+            phase_b(std::true_type{}, st, 1, st, 0, st ^ 1, 1);
+            load_k(min(j + 3, n - 1));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    float lt = lsum + __shfl_xor(lsum, 32);
+    if constexpr (KG == 2) {
+        // group 1's partial result through LDS, lane for lane (both groups hold
+        // the same queries and columns in the same registers)
+        float* X = reinterpret_cast<float*>(smem) + wave * 64 * 32;
+        float* ML = reinterpret_cast<float*>(smem) + 4 * 64 * 32 + wave * 128;
+        __syncthreads();
+        if (grp == 1) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<floatx4*>(X + ((4 * u + q) * 64 + lane) * 4) =
+                        floatx4{o[u][4 * q], o[u][4 * q + 1], o[u][4 * q + 2], o[u][4 * q + 3]};
+            ML[lane] = m;
+            ML[64 + lane] = lt;
+        }
+        __syncthreads();
+        if (grp == 1) return;
+        const float l1 = ML[64 + lane];
+        const float m0 = lt != 0.0f ? m : -INFINITY, m1 = l1 != 0.0f ? ML[lane] : -INFINITY;
+        const float M = fmaxf(m0, m1);
+        const float a0 = m0 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m0 - M) * c);
+        const float a1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m1 - M) * c);
+        lt = a0 * lt + a1 * l1;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const floatx4 x = *reinterpret_cast<const floatx4*>(X + ((4 * u + q) * 64 + lane) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[u][4 * q + e] = a0 * o[u][4 * q + e] + a1 * x[e];
+            }
+    }
+    const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
+    if (a.ostage) {
+        // through LDS; group 1's partials of this wave are read before they are overwritten
+        if constexpr (KG == 1) __syncthreads();  // every wave is done with the stages
+        else __builtin_amdgcn_wave_barrier();
+        const int nrows = qwave >= a.Tq ? 0 : static_cast<int>(min(a.Tq - qwave, 32u));
+        TO* Ob = static_cast<TO*>(a.o) + b * a.so + static_cast<uint64_t>(qwave) * a.ldo + static_cast<uint64_t>(h) * a.hd;
+        store_o_rows<TO>(o, inv, reinterpret_cast<char*>(smem) + wave * 64 * 32 * 4, Ob, nrows, hd, a.ldo, lane);
+        return;
     }
     if (qi >= a.Tq) return;
     TO* Op = static_cast<TO*>(a.o) + b * a.so + static_cast<uint64_t>(qi) * a.ldo + static_cast<uint64_t>(h) * a.hd;
@@ -504,18 +864,13 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
 #pragma unroll
         for (int run = 0; run < 4; ++run) {
             const int d0 = 32 * u + 8 * run + 4 * g;
-            if (VEC && d0 + 4 <= hd) {
-                if constexpr (sizeof(TO) == 4) {
-                    *reinterpret_cast<floatx4*>(Op + d0) =
-                        floatx4{o[u][4 * run] * inv, o[u][4 * run + 1] * inv, o[u][4 * run + 2] * inv, o[u][4 * run + 3] * inv};
-                } else {
-                    *reinterpret_cast<half4*>(Op + d0) = half4_of(o[u][4 * run] * inv, o[u][4 * run + 1] * inv,
-                                                                  o[u][4 * run + 2] * inv, o[u][4 * run + 3] * inv);
-                }
+            if (d0 >= hd) continue;
+            if constexpr (sizeof(TO) == 4) {
+                *reinterpret_cast<floatx4*>(Op + d0) =
+                    floatx4{o[u][4 * run] * inv, o[u][4 * run + 1] * inv, o[u][4 * run + 2] * inv, o[u][4 * run + 3] * inv};
             } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (d0 + e < hd) Op[d0 + e] = static_cast<TO>(o[u][4 * run + e] * inv);
+                *reinterpret_cast<half4*>(Op + d0) = half4_of(o[u][4 * run] * inv, o[u][4 * run + 1] * inv,
+                                                              o[u][4 * run + 2] * inv, o[u][4 * run + 3] * inv);
             }
         }
 }
@@ -544,11 +899,6 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
 // j+1), so one barrier per tile keeps both double buffers race-free. The
 // workgroup has NW waves of 32 queries; blocks are mapped so that the
 // workgroups of one (batch, head) share an XCD (and its L2).
-// RESID: which tiles add P's fp16 residual as a second PV product, at compile
-// time (a runtime test of the flag inside the loop cost non-causal launches
-// 2.4%): kResidNone; kResidDiagonal, a causal launch's diagonal tiles;
-// kResidAll, every tile (MI_ATTN_PREC_SPLIT).
-constexpr int kResidNone = 0, kResidDiagonal = 1, kResidAll = 2;
 // BURST: the burst-ordered loop (below) built for three waves per SIMD
 // (168 registers): a third workgroup per CU for grids of more than two per CU.
 template <typename TO, int NW, int RESID, int BURST = 0>
@@ -1191,11 +1541,33 @@ void launch_f16(const AttnArgs& a, uint32_t batch, hipStream_t s) {
     }
 }
 
+// fp32 inputs on the vector path. Two key groups per workgroup (one 8-wave
+// workgroup per CU) where the last round of two 4-wave workgroups per CU would
+// leave no more than one on each: a grid of W workgroups with (W - 1) mod 2 CUs
+// below the CU count, and at least 512 keys, below which the second group's
+// start and the final addition cost more than it saves. Measured on MI355X, us,
+// two groups / one: 1 x 10 x 2304^2 (180 workgroups) 52.5 / 58.8, 1 x 20 x 1024^2
+// (160) 25.9 / 29.2, 2 x 10 x 4096^2 (640) 274 / 282; the other way round 2 x 20 x
+// 1024^2 (320) 52.7 / 46.8, 2 x 10 x 2304^2 (360) 104 / 99, 1 x 20 x 1024 x 77 9.5 /
+// 8.8. A causal launch carries P's residual on every tile.
+template <typename TO>
+void launch_f32(const AttnArgs& a, uint32_t batch, hipStream_t s) {
+    const uint32_t qtiles = ceil_div(a.Tq, kBQ);
+    const unsigned grid = static_cast<unsigned>(static_cast<uint64_t>(qtiles) * a.heads * batch);
+    const uint32_t cus = cu_count();
+    const bool two = a.Tk >= 512 && (grid - 1) % (2 * cus) < cus;
+    if (a.precise || a.causal) {
+        if (two) attn_f32_kernel<TO, kResidAll, 2><<<grid, 512, 0, s>>>(a, qtiles);
+        else attn_f32_kernel<TO, kResidAll, 1><<<grid, 256, 0, s>>>(a, qtiles);
+    } else {
+        if (two) attn_f32_kernel<TO, kResidNone, 2><<<grid, 512, 0, s>>>(a, qtiles);
+        else attn_f32_kernel<TO, kResidNone, 1><<<grid, 256, 0, s>>>(a, qtiles);
+    }
+}
+
 template <typename TI, typename TO>
-void launch_typed(const AttnArgs& a, uint32_t batch, bool vec, hipStream_t s) {
-    dim3 grid(ceil_div(a.Tq, kBQ), a.heads, batch);
-    if (vec) attn_kernel<TI, TO, true><<<grid, kThreads, 0, s>>>(a);
-    else attn_kernel<TI, TO, false><<<grid, kThreads, 0, s>>>(a);
+void launch_typed(const AttnArgs& a, uint32_t batch, hipStream_t s) {
+    attn_kernel<TI, TO, false><<<dim3(ceil_div(a.Tq, kBQ), a.heads, batch), kThreads, 0, s>>>(a);
 }
 
 // need: when set, only the workspace bytes a split plan would use are stored
@@ -1252,8 +1624,9 @@ int run(const mi_attn_args& x, hipStream_t s, const char* fn, void* ws = nullptr
                      (so * eo) % vout == 0 && (a.hd * ei) % vin == 0;
     // fp16 inputs on the vector path: the pipelined kernel (one workgroup per
     // 64 or 128 queries of one (batch, head), 1-D grid)
-    const bool fast = vec && x.in_dtype == MI_F16 &&
-                      static_cast<uint64_t>(ceil_div(x.Tq, 64u)) * x.heads * x.batch < (1ull << 31);
+    const bool small_grid = static_cast<uint64_t>(ceil_div(x.Tq, 64u)) * x.heads * x.batch < (1ull << 31);
+    const bool fast = vec && x.in_dtype == MI_F16 && small_grid;
+    const bool fast32 = vec && x.in_dtype == MI_F32 && small_grid;
     a.nfull = 0;
     a.pieces = 1;
     a.part = nullptr;
@@ -1279,10 +1652,12 @@ int run(const mi_attn_args& x, hipStream_t s, const char* fn, void* ws = nullptr
     }
     if (fast && x.out_dtype == MI_F16) launch_f16<_Float16>(a, x.batch, s);
     else if (fast) launch_f16<float>(a, x.batch, s);
-    else if (x.in_dtype == MI_F16 && x.out_dtype == MI_F16) launch_typed<_Float16, _Float16>(a, x.batch, vec, s);
-    else if (x.in_dtype == MI_F16) launch_typed<_Float16, float>(a, x.batch, vec, s);
-    else if (x.out_dtype == MI_F16) launch_typed<float, _Float16>(a, x.batch, vec, s);
-    else launch_typed<float, float>(a, x.batch, vec, s);
+    else if (fast32 && x.out_dtype == MI_F16) launch_f32<_Float16>(a, x.batch, s);
+    else if (fast32) launch_f32<float>(a, x.batch, s);
+    else if (x.in_dtype == MI_F16 && x.out_dtype == MI_F16) launch_typed<_Float16, _Float16>(a, x.batch, s);
+    else if (x.in_dtype == MI_F16) launch_typed<_Float16, float>(a, x.batch, s);
+    else if (x.out_dtype == MI_F16) launch_typed<float, _Float16>(a, x.batch, s);
+    else launch_typed<float, float>(a, x.batch, s);
     return check_launch(fn);
 }
 
