@@ -135,8 +135,11 @@ int mi_q8_0_quantize(const float* w, void* blocks, uint64_t n, void* stream);
  * aligned. C must not overlap A, W or bias.
  * Returns MI_OK for M == 0 || N == 0 (nothing to do); K == 0 stores bias/0.
  * Determinism: every entry sums in a fixed order, so a call repeats bit for
- * bit. The entries without a workspace never split K, and every such call
- * gives the same bits whatever tile build runs it. The *_ws entries may split
+ * bit. The entries without a workspace never split K across workgroups, and
+ * every such call gives the same bits whatever tile build runs it (calls of up
+ * to 16 rows, with or without a workspace, sum K in eight interleaved parts
+ * inside a workgroup: the same bits in every entry, another grouping than the
+ * tiles'). The *_ws entries may split
  * K into the caller's workspace (partials summed in split order by a second
  * kernel): bit-identical from run to run, but grouped differently from the
  * unsplit sum (last-bit differences from the entry without a workspace).

@@ -810,6 +810,173 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
                                      kFreshLane ? lane_id() : lane);
 }
 
+// ---- few rows ----------------------------------------------------------------------
+//
+// M <= kFewRows (a step's time-embedding projections: one row per guidance pass).
+// The 64 x 64 tiles spend such a call on a serial chain of K steps in N / 64
+// workgroups, or on two launches. Here a workgroup takes 16 columns and its eight
+// waves the 128-k steps in turn (wave w: steps w, w + 8, ...), each with a partial
+// 16 x 16 tile (v_mfma_f32_16x16x32_f16) that they add at the end through LDS in
+// wave order. K is never split across workgroups, there is no workspace, and every
+// entry (layouts, fp16 A, fp16 output, modes, GEGLU) sums in this one order, so calls
+// that differ in those alone agree bit for bit as they do on the tiles.
+//   * Weights: the lane of column n and quarter c of the wave holds one whole block of
+//     its row (block 4s + c of step s: a load instruction covers 16 rows x 136 bytes),
+//     dequantised straight into four MFMA operands; the A operand takes its k values
+//     in the same order (an MFMA's sum does not care which 32 k it is given as long as
+//     both operands agree).
+//   * A: whole row pieces (a 16-byte load per lane, two fp32 rows or four fp16 rows
+//     per instruction), as fp16 through a wave-private LDS tile; rows past M read out
+//     of range. Loading the operands lane by lane instead (eight loads per step, most
+//     lanes out of range) cost 1.1 us of 5.2 at 2x1280x1280: the load path charges an
+//     instruction for its 64 lanes whatever they read.
+// Bound by one memory round trip and the launch: two steps of loads per wave are in
+// flight before the first MFMA. Measured on MI355X, us, against the 64 x 64 tiles with
+// their K split and reduce pass / without a workspace: 2x1280x1280 7.5 / 11.2 -> 3.7,
+// 8x1280x2816 8.1 / 21.6 -> 5.9, 16x1280x1280 7.9 / 11.3 -> 4.4, 16x10240x1280 12.2 /
+// 11.4 -> 9.6, 2x1280x5120 9.4 / 36.9 -> 5.3 (kFewRows: the 16 rows of the MFMA).
+constexpr uint32_t kFewRows = 16;
+
+// MA: A rows the loads cover (4 or kFewRows).
+template <int WK, int EPI, bool AH, int MA>
+__global__ __launch_bounds__(512) void gemm_q8_rows_kernel(GemmArgs a) {
+    constexpr int NWV = 8, AE = AH ? 2 : 4;                 // waves, bytes per A element
+    constexpr int AL = MA * 128 * AE / 1024;                // A loads per step (1 KB each)
+    constexpr int LPR = 128 * AE / 16;                      // lanes per A row piece
+    constexpr int LDA = 136;                                // halves per staged A row (16-byte pad)
+    constexpr int kRed = 20;                                // floats per partial row (16-byte pad)
+    constexpr int kCols = EPI == kEpiGeglu ? 8 : 16;        // outputs per row of a workgroup
+    constexpr uint32_t kPast = 0x80000000u;                 // an offset past every record (few_rows)
+    static_assert(AL >= 1, "a load covers at least one whole row");
+    __shared__ __attribute__((aligned(16))) _Float16 As[NWV][kFewRows * LDA];
+    __shared__ __attribute__((aligned(16))) float red[NWV][kFewRows][kRed];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t l16 = lane & 15, c = lane >> 4;
+    const uint32_t n0 = blockIdx.x * kCols;
+    // GEGLU: eight value rows, then the gate rows of the same outputs
+    const uint32_t o = EPI == kEpiGeglu ? min(n0 + (l16 & 7u), a.F - 1u) : 0u;
+    const uint32_t n = EPI == kEpiGeglu ? ((l16 & 8u) ? a.F + o : o) : min(n0 + l16, a.N - 1);
+    const uint32_t nblk = a.K / 32, nsteps = (nblk + 3) / 4;
+
+    const __amdgpu_buffer_rsrc_t rA = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(reinterpret_cast<const char*>(a.A) + static_cast<uint64_t>(blockIdx.z) * a.sA * AE), 0,
+        static_cast<int>(((a.M - 1) * a.lda + a.K) * AE), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(a.W), 0, static_cast<int>(WK == kBlocks34 ? (a.N * a.rowbytes + 15u) & ~15u : a.N * a.K),
+        0x00020000);
+    const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(WK == kSplit ? a.scales : a.A), 0, WK == kSplit ? static_cast<int>(a.N * nblk * 4) : 0,
+        0x00020000);
+    // blocks: a 36-byte window at the block's 4-byte-aligned start; a step moves 136
+    // bytes, so the block's place in its window (0 or 2 bytes) is the lane's own
+    const uint32_t w0 = WK == kBlocks34 ? n * a.rowbytes + c * 34 : n * a.K + c * 32;
+    const uint32_t qsel = (w0 & 2u) ? 0x07060504u : 0x05040302u, dsel = (w0 & 2u) ? 0x0c0c0302u : 0x0c0c0100u;
+    const uint32_t arow = lane / LPR, acol = (lane % LPR) * (16 / AE);  // row and column of the first load
+
+    floatx4 areg[2][AL];
+    uint32_t wreg[2][9];
+    auto load = [&](uint32_t s, auto SET) {
+        constexpr int r = decltype(SET)::value;
+        const uint32_t k = 128 * s + acol;  // K is a multiple of 32: a 16-byte unit is whole or past K
+#pragma unroll
+        for (int i = 0; i < AL; ++i) {
+            const uint32_t row = arow + i * (64 / LPR);
+            areg[r][i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                         rA, row < a.M && k < a.K ? (row * a.lda + k) * AE : kPast, 0, 0));
+        }
+        const bool in = 4 * s + c < nblk;  // past K: zeros for both operands
+        const uint32_t wo = !in ? kPast : WK == kBlocks34 ? (w0 & ~3u) + 136 * s : w0 + 128 * s;
+        const auto x0 = __builtin_amdgcn_raw_buffer_load_b128(rW, wo, 0, 0);
+        const auto x1 = __builtin_amdgcn_raw_buffer_load_b128(rW, wo + 16, 0, 0);
+        wreg[r][8] = WK == kBlocks34 ? __builtin_amdgcn_raw_buffer_load_b32(rW, wo + 32, 0, 0)
+                                     : __builtin_amdgcn_raw_buffer_load_b32(rS, in ? (n * nblk + 4 * s + c) * 4 : kPast, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            wreg[r][e] = x0[e];
+            wreg[r][4 + e] = x1[e];
+        }
+    };
+    floatx4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    _Float16* const At = As[wave];
+    auto compute = [&](auto SET) {
+        constexpr int r = decltype(SET)::value;
+        const uint32_t* x = wreg[r];
+#pragma unroll
+        for (int i = 0; i < AL; ++i) {
+            _Float16* dst = At + (arow + i * (64 / LPR)) * LDA + acol;
+            if constexpr (AH) {
+                *reinterpret_cast<half8*>(dst) = __builtin_bit_cast(half8, areg[r][i]);
+            } else {
+                *reinterpret_cast<half4*>(dst) =
+                    half4{static_cast<_Float16>(areg[r][i][0]), static_cast<_Float16>(areg[r][i][1]),
+                          static_cast<_Float16>(areg[r][i][2]), static_cast<_Float16>(areg[r][i][3])};
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            half8 wf;
+            if constexpr (WK == kBlocks34) {
+                const _Float16 d =
+                    __builtin_bit_cast(_Float16, static_cast<uint16_t>(__builtin_amdgcn_perm(x[0], x[0], dsel)));
+                wf = dequant8_f16(__builtin_amdgcn_perm(x[2 * j + 1], x[2 * j], qsel),
+                                  __builtin_amdgcn_perm(x[2 * j + 2], x[2 * j + 1], qsel), d);
+            } else {
+                const float sc = __builtin_bit_cast(float, x[8]);
+                wf = dequant8_f32(x[2 * j], x[2 * j + 1], sc, sc);
+            }
+            // rows past MA hold nothing: they repeat the others and feed columns never stored
+            const half8 af = *reinterpret_cast<const half8*>(At + (l16 % MA) * LDA + 32 * c + 8 * j);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf, af, acc, 0, 0, 0);  // lane: row m = l16 of C, columns 4c + r
+        }
+        __builtin_amdgcn_wave_barrier();  // every read of this step precedes the next step's writes
+    };
+    using S0 = std::integral_constant<int, 0>;
+    using S1 = std::integral_constant<int, 1>;
+    load(wave, S0{});
+    load(wave + NWV, S1{});
+    for (uint32_t s = wave; s < nsteps; s += 2 * NWV) {
+        compute(S0{});
+        load(s + 2 * NWV, S0{});
+        if (s + NWV < nsteps) compute(S1{});
+        load(s + 3 * NWV, S1{});
+    }
+    if (l16 < a.M) *reinterpret_cast<floatx4*>(&red[wave][l16][4 * c]) = acc;
+    __syncthreads();
+    const uint32_t m = tid / kCols, col = tid % kCols, out = n0 + col;
+    if (m >= a.M || out >= (EPI == kEpiGeglu ? a.F : a.N)) return;
+    auto total = [&](uint32_t i) {
+        float v = red[0][m][i];
+#pragma unroll
+        for (int w = 1; w < NWV; ++w) v += red[w][m][i];
+        return v;
+    };
+    float v = total(col);
+    if constexpr (EPI == kEpiGeglu) {
+        const float bv = a.bias ? a.bias[out] : 0.0f, bg = a.bias ? a.bias[a.F + out] : 0.0f;
+        v = (v + bv) * gelu_erf(total(8 + col) + bg);
+    } else if (a.bias && (EPI == kEpiResidual || a.mode == 0)) {
+        v += a.bias[out];
+    }
+    if (a.out_half) {
+        // one RNE rounding of the fp32 value (as in store_tiles)
+        asm volatile("" : "+v"(v));
+        reinterpret_cast<_Float16*>(a.C)[static_cast<uint64_t>(m) * a.ldc + out] = static_cast<_Float16>(v);
+        return;
+    }
+    float* cp = a.C + static_cast<uint64_t>(blockIdx.z) * a.sC + static_cast<uint64_t>(m) * a.ldc + out;
+    if (EPI == kEpiResidual || (EPI == kEpiPlain && a.mode != 0)) *cp += v;
+    else *cp = v;
+}
+
+// The few-rows kernel takes a call: whole blocks, weights below 2 GiB (its
+// out-of-range offset), no pinned tile build.
+bool few_rows(uint32_t M, uint32_t N, uint32_t K) {
+    return M <= kFewRows && K % 32 == 0 && static_cast<uint64_t>(N) * (K / 32) * 34 < (uint64_t(1) << 31) - 16 &&
+           tuning().gemm_cfg.load(std::memory_order_relaxed) < 0;
+}
+
 // K == 0: C[m, n] = bias[n] (or 0) in mode 0, C[m, n] += bias[n] in mode 2.
 __global__ __launch_bounds__(256) void gemm_fill_kernel(float* C, const float* bias, uint32_t M, uint32_t N,
                                                         uint32_t ldc, uint64_t sC, uint32_t add) {
@@ -1117,6 +1284,7 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, bool allow_split
                                : 1u;
         return p;
     }
+    if (few_rows(M, N, K)) return p;  // no tiles, no split (gemm_q8_rows_kernel)
     auto tiles = [&](uint32_t bm, uint32_t bn) {
         return static_cast<uint64_t>(ceil_div(M, bm)) * ceil_div(N, bn) * batch;
     };
@@ -1167,6 +1335,12 @@ Plan plan_for(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, const void* ws
 
 template <int WK, int EPI = kEpiPlain, bool AH = false>
 void dispatch(const GemmArgs& a, uint32_t batch, const Plan& p, float* ws, hipStream_t s) {
+    if (few_rows(a.M, a.N, a.K)) {
+        const dim3 grid(EPI == kEpiGeglu ? ceil_div(a.F, 8) : ceil_div(a.N, 16), 1, batch);
+        if (a.M <= 4) gemm_q8_rows_kernel<WK, EPI, AH, 4><<<grid, 512, 0, s>>>(a);
+        else gemm_q8_rows_kernel<WK, EPI, AH, 16><<<grid, 512, 0, s>>>(a);
+        return;
+    }
     if (a.K % 64 != 0) launch_general<WK, EPI, AH>(a, batch, p.splits, ws, s);
     else launch<WK, EPI, AH>(p.cfg, a, batch, p.splits, ws, s);
 }

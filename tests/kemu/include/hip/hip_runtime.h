@@ -267,6 +267,43 @@ inline f16v mfma_32x32x16_f16(h8 a, h8 b, f16v c, int cbsz, int abid, int blgp) 
     return d;
 }
 
+// v_mfma_f32_16x16x32_f16: A 16x32, B 32x16. Lane l supplies A row l % 16 and B
+// column l % 16, k = 8 (l / 16) + 0..7; D / C: lane l, register r holds row
+// 4 (l / 16) + r, column l % 16.
+typedef float f4v __attribute__((ext_vector_type(4)));
+struct Mfma16In {
+    h8 a, b;
+    f4v c;
+};
+inline void mfma16_fn(const unsigned char (*ins)[256], unsigned char (*outs)[256], const void*) {
+    float A[16][32], B[32][16], Cm[16][16];
+    for (int l = 0; l < 64; ++l) {
+        Mfma16In x;
+        std::memcpy(&x, ins[l], sizeof x);
+        for (int e = 0; e < 8; ++e) {
+            A[l % 16][8 * (l / 16) + e] = static_cast<float>(x.a[e]);
+            B[8 * (l / 16) + e][l % 16] = static_cast<float>(x.b[e]);
+        }
+        for (int r = 0; r < 4; ++r) Cm[4 * (l / 16) + r][l % 16] = x.c[r];
+    }
+    for (int l = 0; l < 64; ++l) {
+        f4v d;
+        for (int r = 0; r < 4; ++r) {
+            double s = Cm[4 * (l / 16) + r][l % 16];
+            for (int k = 0; k < 32; ++k) s += static_cast<double>(A[4 * (l / 16) + r][k]) * B[k][l % 16];
+            d[r] = static_cast<float>(s);
+        }
+        std::memcpy(outs[l], &d, sizeof d);
+    }
+}
+inline f4v mfma_16x16x32_f16(h8 a, h8 b, f4v c, int cbsz, int abid, int blgp) {
+    if (cbsz || abid || blgp) die("mfma: broadcast controls are not emulated");
+    const Mfma16In x{a, b, c};
+    f4v d;
+    wave_op("mfma_f32_16x16x32_f16", &x, sizeof x, &d, sizeof d, mfma16_fn, nullptr);
+    return d;
+}
+
 struct DppCtl {
     int ctrl;
 };
@@ -457,6 +494,7 @@ inline T __shfl_xor(T v, int mask, int width = 64) {
 #define __builtin_amdgcn_raw_buffer_load_b128 ::kemu::buffer_load_b128
 #define __builtin_amdgcn_raw_buffer_store_b32 ::kemu::buffer_store_b32
 #define __builtin_amdgcn_mfma_f32_32x32x16_f16 ::kemu::mfma_32x32x16_f16
+#define __builtin_amdgcn_mfma_f32_16x16x32_f16 ::kemu::mfma_16x16x32_f16
 #define __builtin_amdgcn_mov_dpp ::kemu::mov_dpp
 #define __builtin_amdgcn_readfirstlane ::kemu::readfirstlane
 #define __builtin_amdgcn_mbcnt_lo ::kemu::mbcnt_lo
