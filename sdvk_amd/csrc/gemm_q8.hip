@@ -380,7 +380,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     constexpr int A_IT = A_UNITS / NT;
     constexpr int W_UNITS = BN * BK / 8;          // (row, 8-k group) per step
     constexpr int W_IT = W_UNITS / NT;
-    // 34-byte blocks with two blocks per step: one whole block per lane (three
+    // Two or more blocks per step: one whole block per lane (three
     // loads for 32 weights). Block wb of a step is weight row wb / KB, block
     // column wb % KB: the KB blocks of a row (its 68 contiguous bytes of the
     // step) sit on adjacent lanes, so one load instruction of a wave touches
@@ -389,7 +389,13 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     // load path this way against 1209 with a wave's lanes on 64 rows (a
     // load-only probe of the step on MI355X; 16 rows, the four blocks of two
     // steps, take 607 but gained nothing in the kernel).
-    constexpr bool WBLK = WK == kBlocks34 && KB == 2 && !KTAIL;
+    // Four blocks per step (KB = 4, the 64x64 tile at K % 128 == 0): 16 rows per
+    // instruction, every block loaded once, half the barriers: 1152x1280x1280 16.1 ->
+    // 14.8 us, 1152x1280x5120 66 -> 52, 2304x640x2560 33 -> 25 (MI355X, fp32 A).
+    // The split layout loads a block's 32 payload bytes and its scale the same way
+    // (three loads per block; one payload load and one scale load per 8 weights
+    // before): 9216x1280x1280 50.8 -> 46.6 us, 2048x10240x1280 76 -> 67.5.
+    constexpr bool WBLK = (KB == 2 || KB == 4) && !KTAIL;
     constexpr int W_BLOCKS = BN * KB;
     constexpr int WB_IT = (W_BLOCKS + NT - 1) / NT;
     // Twice as many threads as blocks in a 4-wave workgroup (the 64x64 and
@@ -403,9 +409,6 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     // 128x128 tile's weights in the probe, against 674 with every block loaded
     // twice.
     constexpr bool WHALF = WBLK && 2 * W_BLOCKS == NT && NT == 256;
-    // Buffer-load fast path: two blocks per step keep each lane's byte
-    // alignment fixed (68 = 0 mod 4), so the step advance is a scalar offset.
-    constexpr bool FAST = KB == 2 && !KTAIL;
     static_assert(A_UNITS % NT == 0 && W_UNITS % NT == 0, "staging must divide evenly");
     static_assert(FM >= 1 && FN >= 1, "wave tile below 32x32");
 
@@ -452,7 +455,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     // 34-byte layout: records up to W's 16-byte-aligned end (the documented
     // read extent); the range check zeroes whole dwords only past that.
     const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(a.W), 0, WK == kBlocks34 ? static_cast<int>((a.N * a.rowbytes + 15u) & ~15u) : -1,
+        const_cast<uint8_t*>(a.W), 0, static_cast<int>(WK == kBlocks34 ? (a.N * a.rowbytes + 15u) & ~15u : a.N * a.K),
         0x00020000);
     const __amdgpu_buffer_rsrc_t rS =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(WK == kSplit ? a.scales : a.A), 0, -1, 0x00020000);
@@ -491,29 +494,26 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     uint32_t w0_[PF][W_IT], w1_[PF][W_IT], w2_[PF][W_IT], wd_[PF][W_IT];
     float ws0_[PF][W_IT], ws1_[PF][W_IT];
     // 34-byte layout: lanes whose 8 q bytes start 2 mod 4 read one more dword
-    // and funnel-shift by 16 bits; in the fast path the shift is fixed per lane.
+    // and funnel-shift by 16 bits.
     uint32_t w_sh[PF][W_IT];
-#pragma unroll
-    for (int i = 0; i < W_IT; ++i)
-#pragma unroll
-        for (int r = 0; r < PF; ++r) w_sh[r][i] = (w_off[i] & 2u) * 8u;
     // Whole-block staging: the 36-byte window at the block's 4-byte-aligned
-    // start; the row stride is 0 mod 4 (K % 64 == 0) and a step advances 68
-    // bytes, so a block's position inside its window (0 or 2 bytes) is fixed
-    // for the lane. v_perm selectors pick d and the eight q dwords for either.
+    // start; the row stride is 0 mod 4 (K % 64 == 0) and a step advances 34 KB
+    // bytes (0 mod 4), so a block's position inside its window (0 or 2 bytes) is
+    // fixed for the lane. (Split layout: the block's 32 bytes and its scale.) v_perm selectors pick d and the eight q dwords for either.
     // Threads past the step's W_BLOCKS blocks still issue the loads (out of
     // range: zeros, no memory access) and store nothing: a load under a branch
     // makes the compiler's wait counts assume it was skipped, so every later
     // wait would also retire the loads of the step just issued.
-    uint32_t wb_off[WB_IT], wb_qsel[WB_IT], wb_dsel[WB_IT];
+    uint32_t wb_off[WB_IT], wb_qsel[WB_IT], wb_dsel[WB_IT], wb_sc[WB_IT];
     uint32_t wbx_[PF][WB_IT][9];
 #pragma unroll
     for (int i = 0; i < WB_IT; ++i) {
         const int wb = (tid + i * NT) % W_BLOCKS;
         const uint32_t n = EPI == kEpiGeglu ? geglu_wrow(n0, wb / KB, a.F) : min(n0 + wb / KB, a.N - 1);
-        const uint32_t byte = n * a.rowbytes + (wb % KB) * 34;
+        const uint32_t byte = WK == kBlocks34 ? n * a.rowbytes + (wb % KB) * 34 : n * a.K + (wb % KB) * 32;
         // past the step's blocks: out of range, so the load returns zeros and touches no memory
-        wb_off[i] = (!WHALF && W_BLOCKS % NT != 0 && tid + i * NT >= W_BLOCKS) ? 0x80000000u : byte & ~3u;
+        wb_off[i] = (!WHALF && W_BLOCKS % NT != 0 && tid + i * NT >= W_BLOCKS) ? 0xffffff00u : byte & ~3u;
+        wb_sc[i] = (n * (a.K / 32) + wb % KB) * 4;
         wb_qsel[i] = (byte & 2u) ? 0x07060504u : 0x05040302u;  // bytes 4..7 or 2..5 of (x[j+1]:x[j])
         wb_dsel[i] = (byte & 2u) ? 0x0c0c0302u : 0x0c0c0100u;  // bytes 2,3 or 0,1 of x[0]; 0x0c = zero
     }
@@ -534,12 +534,13 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
             }
         }
         if constexpr (WBLK) {
-            const uint32_t soff = ks * (KB * 34);
+            const uint32_t soff = ks * (KB * (WK == kBlocks34 ? 34 : 32));
 #pragma unroll
             for (int i = 0; i < WB_IT; ++i) {
                 const auto x0 = __builtin_amdgcn_raw_buffer_load_b128(rW, wb_off[i], soff, 0);
                 const auto x1 = __builtin_amdgcn_raw_buffer_load_b128(rW, wb_off[i] + 16, soff, 0);
-                wbx_[rs][i][8] = __builtin_amdgcn_raw_buffer_load_b32(rW, wb_off[i] + 32, soff, 0);
+                wbx_[rs][i][8] = WK == kBlocks34 ? __builtin_amdgcn_raw_buffer_load_b32(rW, wb_off[i] + 32, soff, 0)
+                                                 : __builtin_amdgcn_raw_buffer_load_b32(rS, wb_sc[i], ks * (KB * 4), 0);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     wbx_[rs][i][e] = x0[e];
@@ -551,22 +552,15 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
         for (int i = 0; i < (WBLK ? 0 : W_IT); ++i) {
             if constexpr (WK == kBlocks34) {
                 const uint32_t soff = ks * (KB * 34);
-                const uint32_t addr = FAST ? w_off[i] : w_off[i] + soff;
+                const uint32_t addr = w_off[i] + soff;
                 const uint32_t base = addr & ~3u;
-                const uint32_t so = FAST ? soff : 0u;
-                const auto w01 = __builtin_amdgcn_raw_buffer_load_b64(rW, base, so, 0);
+                const auto w01 = __builtin_amdgcn_raw_buffer_load_b64(rW, base, 0, 0);
                 w0_[rs][i] = w01[0];
                 w1_[rs][i] = w01[1];
                 // third dword only matters when shifted; otherwise re-read the second
-                w2_[rs][i] = __builtin_amdgcn_raw_buffer_load_b32(rW, base + ((addr & 2u) ? 8u : 4u), so, 0);
-                wd_[rs][i] = __builtin_amdgcn_raw_buffer_load_b16(rW, FAST ? w_aux[i] : w_aux[i] + soff, so, 0);
-                if constexpr (!FAST) w_sh[rs][i] = (addr & 2u) * 8u;  // shift of this set's step
-            } else if constexpr (FAST) {
-                const auto w01 = __builtin_amdgcn_raw_buffer_load_b64(rW, w_off[i], ks * BK, 0);
-                w0_[rs][i] = w01[0];
-                w1_[rs][i] = w01[1];
-                ws0_[rs][i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rS, w_aux[i], ks * KB * 4, 0));
-                ws1_[rs][i] = ws0_[rs][i];
+                w2_[rs][i] = __builtin_amdgcn_raw_buffer_load_b32(rW, base + ((addr & 2u) ? 8u : 4u), 0, 0);
+                wd_[rs][i] = __builtin_amdgcn_raw_buffer_load_b16(rW, w_aux[i] + soff, 0, 0);
+                w_sh[rs][i] = (addr & 2u) * 8u;  // shift of this set's step
             } else {
                 const uint32_t k = ks * BK + w_k[i];
                 const uint64_t f = static_cast<uint64_t>(w_off[i]) + static_cast<uint64_t>(ks) * BK;
@@ -604,37 +598,49 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
                 *reinterpret_cast<half4*>(&As[st][(f / (BK / 4)) * LDK + (f % (BK / 4)) * 4]) = h;
             }
         }
+        // eight weights of block i from dword j on (q dwords j, j + 1)
+        auto dequant = [&](int i, uint32_t lo, uint32_t hi) {
+            const uint32_t* x = wbx_[rs][i];
+            if constexpr (WK == kBlocks34) {
+                return dequant8_f16(lo, hi, __builtin_bit_cast(_Float16, static_cast<uint16_t>(
+                                                __builtin_amdgcn_perm(x[0], x[0], wb_dsel[i]))));
+            } else {
+                const float sc = __builtin_bit_cast(float, x[8]);
+                return dequant8_f32(lo, hi, sc, sc);
+            }
+        };
         if constexpr (WHALF) {
             const uint32_t* x = wbx_[rs][0];
             const bool hi = tid >= W_BLOCKS;  // wave-uniform: W_BLOCKS is a multiple of 64
-            uint32_t xs[5];
+            constexpr int NX = WK == kBlocks34 ? 5 : 4;
+            uint32_t xs[NX], q[4];
 #pragma unroll
-            for (int j = 0; j < 5; ++j) xs[j] = hi ? x[4 + j] : x[j];
-            const _Float16 d = __builtin_bit_cast(
-                _Float16, static_cast<uint16_t>(__builtin_amdgcn_perm(x[0], x[0], wb_dsel[0])));
-            uint32_t q[4];
+            for (int j = 0; j < NX; ++j) xs[j] = hi ? x[4 + j] : x[j];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) q[j] = __builtin_amdgcn_perm(xs[j + 1], xs[j], wb_qsel[0]);
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (WK == kBlocks34) q[j] = __builtin_amdgcn_perm(xs[j + 1], xs[j], wb_qsel[0]);
+                else q[j] = xs[j];
+            }
             const int wb = hi ? tid - W_BLOCKS : tid;
             _Float16* dst = &Ws[st][(wb / KB) * LDK + (wb % KB) * 32 + (hi ? 16 : 0)];
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-                *reinterpret_cast<half8*>(dst + 8 * j) = dequant8_f16(q[2 * j], q[2 * j + 1], d);
+            for (int j = 0; j < 2; ++j) *reinterpret_cast<half8*>(dst + 8 * j) = dequant(0, q[2 * j], q[2 * j + 1]);
         } else if constexpr (WBLK) {
 #pragma unroll
             for (int i = 0; i < WB_IT; ++i) {
                 const int wb = tid + i * NT;
                 if (W_BLOCKS % NT == 0 || wb < W_BLOCKS) {
                     const uint32_t* x = wbx_[rs][i];
-                    const _Float16 d = __builtin_bit_cast(
-                        _Float16, static_cast<uint16_t>(__builtin_amdgcn_perm(x[0], x[0], wb_dsel[i])));
                     uint32_t q[8];
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) q[j] = __builtin_amdgcn_perm(x[j + 1], x[j], wb_qsel[i]);
+                    for (int j = 0; j < 8; ++j) {
+                        if constexpr (WK == kBlocks34) q[j] = __builtin_amdgcn_perm(x[j + 1], x[j], wb_qsel[i]);
+                        else q[j] = x[j];
+                    }
                     _Float16* dst = &Ws[st][(wb / KB) * LDK + (wb % KB) * 32];
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        *reinterpret_cast<half8*>(dst + 8 * j) = dequant8_f16(q[2 * j], q[2 * j + 1], d);
+                        *reinterpret_cast<half8*>(dst + 8 * j) = dequant(i, q[2 * j], q[2 * j + 1]);
                 }
             }
         }
@@ -1237,7 +1243,10 @@ void launch(int cfg, const GemmArgs& a, uint32_t batch, uint32_t splits, float* 
             else
                 launch_cfg<256, 256, 4, 2, 2, WK, false, 1, EPI, true, AH>(a, batch, splits, ws, s);
             break;
-        default: launch_cfg<64, 64, 2, 2, 2, WK, false, 2, EPI, true, AH>(a, batch, splits, ws, s); break;
+        default:
+            if (a.K % 128 == 0) launch_cfg<64, 64, 2, 2, 4, WK, false, 2, EPI, true, AH>(a, batch, splits, ws, s);
+            else launch_cfg<64, 64, 2, 2, 2, WK, false, 2, EPI, true, AH>(a, batch, splits, ws, s);
+            break;
     }
 }
 
