@@ -176,9 +176,8 @@ int mi_gemm_nt_q8_0_ws(const float* A, const void* W, const float* bias, float* 
  * K-split partials go to a scratch array inside the library, one per GPU,
  * of MI_GEMM_NOALLOC_SCRATCH_BYTES, held until the process ends. A shape whose
  * plan needs more scratch than that returns MI_ERR_UNSUPPORTED (no shape does
- * under the built-in tile rules: they split only grids of fewer than 256
- * 128 x 128 tiles, into at most 512 / tiles parts, or fewer than 512 64 x 64
- * tiles into about 256 workgroups, at most 32 MiB of partials). Calls on one GPU share
+ * under the built-in tile rules: a split grid is at most 256 workgroups of
+ * 256 x 128, 128 x 128 or 64 x 64 tiles, so at most 32 MiB of partials). Calls on one GPU share
  * the scratch: calls that overlap on one GPU (unordered streams) race, so
  * order them (one stream). Calls no hipMalloc / hipFree. The scratch's device
  * address is looked up once per GPU (hipGetSymbolAddress, which may load the

@@ -1265,24 +1265,68 @@ struct Plan {
     uint32_t splits;
 };
 
-// Picks the tile and K split for a shape (rules from per-shape sweeps of every
-// tile build on MI355X over the SDXL shapes, timed interleaved): the 192x256
-// tile (8 waves, one workgroup per CU) where it yields a wave or more of
-// long-K tiles over more than 640 columns (at N = 640 the 128x128 tile is
-// faster: 8192x640x2560 61.6 vs 66.0 us), or 256x128 where that fills more of
-// a single round; among the grids of at least 160 128x128 tiles, 256x128 (8
-// waves, ping-pong) where it makes 160 tiles or more, else 128x128 (4 waves,
-// two workgroups per CU), as 8 waves of 32x64 when the grid has fewer tiles
-// than CUs and no K split (one workgroup per CU: two waves per SIMD instead
-// of one; 2048x1280x1280 17.6 vs 21.8 us, 2048x1280x5120 unsplit 60.5 vs
-// 89.5); 64x64 for the rest.
-// With a workspace (allow_split), long-K (>= 4096) 128x128 grids of fewer
-// tiles than CUs run as 256x128 tiles (8 waves) with K split into the most
-// parts (>= 1024 k each) that keep one round (2048x1280x5120: 80 tiles x 3 =
-// 240 workgroups, 52.3 us against 54.1 us for 128x128 tiles in 3 parts with
-// fp32 A and 45.6 against 48.6 with fp16 A; 128x128 in 3 parts had beaten 2
-// and 4 parts, 55.2 against 67.7 and 69.4 us), and small 64x64 grids split K
-// until ~256 workgroups run.
+// Picks the tile and K split for a shape. Rules from sweeps of every tile build on
+// MI355X over the SDXL layers at 512 to 1024 pixels a side, timed interleaved, on
+// weights and activations of full entropy (constant data runs up to a quarter faster:
+// less power, higher clocks). us, fp32 A:
+//   * 192x256 (8 waves, one workgroup per CU) where it yields 120 tiles or more of
+//     long K over more than 640 columns (at N = 640 the 128x128 tile is faster:
+//     8192x640x2560 61.6 vs 66.0), or 256x128 where that fills more of a single
+//     round (the block's joint Q/K/V 2048x3840x1280: 240 against 165 tiles, 30.9
+//     against 32.7 with fp16 A);
+//   * grids that fit one round of two 64x64 tiles per CU (512) take those:
+//     1600x1280x1280 (500 tiles) 16.6 vs 18.3 for 128x128, 576x1280x1280 (180) 11.2
+//     vs 17.0;
+//   * larger ones that fit one round of 128x128 tiles take those as eight waves of
+//     32x64 (one workgroup per CU: two waves per SIMD): 3952x640x640 (620 tiles of
+//     64x64, 155 of 128x128) 11.8 vs 14.8, 1976x1280x1280 18.5 vs 24.0, 3952x640x2560
+//     33.5 vs 40.7;
+//   * the rest 256x128 (8 waves, ping-pong): 7904x640x2560 (310 tiles of 128x128, 155
+//     of 256x128) 49.5 against 61.8 (128x128, 4 waves) and 57.7 (8 waves), 7904x640x640
+//     19.4 against 21.0 and 20.5, 8192x5120x640 90.5 against 91.7.
+// With a workspace (allow_split):
+//   * up to 128 64x64 tiles split K (powers of two, >= 128 k each) until about 256
+//     workgroups run: 154x1280x2048 (60 tiles x 4) 10.3 vs 15.6 unsplit. At 180 tiles
+//     two splits lose (576x1280x1280 14.1 vs 11.2 unsplit: the second launch and the
+//     partials cost more than half of a short K);
+//   * K >= 2560 on grids of up to 256 128x128 tiles: long_k_plan below.
+//
+// long_k_plan: the cheapest of the builds that fit one round, each with K split into
+// the most parts (>= 640 k) that still do. A 64-k step of a lone workgroup per CU takes
+// 0.42 us on 64x64 tiles (0.65 with two per CU), 0.73 on 128x128 (8 waves), 1.05 on
+// 256x128, on top of 1.5 / 4 / 4 us per launch; partial planes cost their write and
+// read at 5 TB/s and a second launch (3.5 us). Measured against the unsplit tiles /
+// the same in two K parts (fp32 A, us): 576x1280x5120 in 5 parts of 128x128 23.3 vs
+// 33.5 / 32.1, 988x1280x5120 in 3 30.7 vs 50.5 / 45.6, 1152x1280x5120 in 5 of 256x128
+// 35.3 vs 52.6 / 47.7, 2048x1280x5120 in 3 of 256x128 48.8 vs 62.0 (128x128);
+// 1024x640x2560 stays on 64x64 (18.3; with fp16 A 15.4 vs 17.4 split), 4608x640x2560 on
+// 128x128 (34.0 vs 36.8 in 2 of 256x128).
+Plan long_k_plan(uint64_t t64, uint64_t t128, uint64_t t256, uint32_t K, uint64_t outputs) {
+    const struct {
+        int cfg;
+        uint64_t tiles;
+        double step_us, launch_us;
+        bool split;
+    } builds[] = {{kC64x64, t64, t64 <= kCUs ? 0.42 : 0.65, 1.5, false},
+                  {kC128x128W8, t128, 0.73, 4.0, true},
+                  {kC256x128, t256, 1.05, 4.0, true}};
+    const uint32_t steps = K / 64;
+    Plan best{kC128x128W8, 1};
+    double best_us = 1e300;
+    for (const auto& c : builds) {
+        if (c.tiles > (c.split ? kCUs : 2 * kCUs)) continue;
+        const uint32_t splits =
+            c.split ? static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(kCUs / c.tiles, K / 640))) : 1;
+        double us = c.launch_us + ceil_div(steps, splits) * c.step_us;
+        if (splits > 1) us += 3.5 + static_cast<double>(splits) * static_cast<double>(outputs) * 8 / 5e6;
+        if (us < best_us) {
+            best_us = us;
+            best = Plan{c.cfg, splits};
+        }
+    }
+    return best;
+}
+
 Plan choose(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, bool allow_split) {
     Plan p{kC64x64, 1};
     // mi_tuning_set("gemm_cfg", "<cfg>[:<splits>]") pins a build (tuning sweeps, tests)
@@ -1299,31 +1343,15 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, bool allow_split
     };
     const uint64_t t192 = tiles(192, 256), t128 = tiles(128, 128), t64 = tiles(64, 64), t256 = tiles(256, 128);
     if (t192 >= 120 && K >= 1280 && N > 640) {
-        // under one round, 256x128 tiles fill more CUs where they still fit one
-        // (the block's joint Q/K/V 2048x3840x1280: 240 against 165 tiles, 30.9
-        // against 32.7 us with fp16 A)
         p.cfg = t192 < kCUs && t256 > t192 && t256 <= kCUs ? kC256x128 : kC192x256;
-    } else if (t128 >= 160) {
-        p.cfg = kC128x128;
-        if (t256 >= 160) {
-            // grids of at least 160 256x128 tiles: the 8-wave ping-pong build
-            // (8192x640x2560 48.4 vs 50.9 us, 8192x640x640 17.1 vs 17.8,
-            // 8192x5120x640 90.5 vs 91.7; with fp16 A 5-9% faster)
-            p.cfg = kC256x128;
-        } else if (allow_split && t128 < kCUs && K >= 4096) {
-            p.cfg = kC256x128;
-            p.splits = static_cast<uint32_t>(std::max<uint64_t>(2, std::min<uint64_t>(kCUs / t256, K / 1024)));
-        } else if (t128 < kCUs) {
-            p.cfg = kC128x128W8;
-        }
-    } else {
-        p.cfg = kC64x64;
-        if (allow_split && t64 < 2 * kCUs) {
-            const uint64_t want = (kCUs + t64 - 1) / t64;
-            uint32_t sp = 1;
-            while (sp * 2 <= want && sp * 2 * 128 <= K) sp *= 2;
-            p.splits = sp;
-        }
+        return p;
+    }
+    p.cfg = t128 > kCUs ? kC256x128 : t64 > 2 * kCUs ? kC128x128W8 : kC64x64;
+    if (!allow_split || t128 > kCUs) return p;
+    if (K >= 2560) return long_k_plan(t64, t128, t256, K, static_cast<uint64_t>(M) * N * batch);
+    if (p.cfg == kC64x64 && t64 <= kCUs / 2) {
+        const uint64_t want = (kCUs + t64 - 1) / t64;
+        while (p.splits * 2 <= want && p.splits * 2 * 128 <= K) p.splits *= 2;
     }
     return p;
 }

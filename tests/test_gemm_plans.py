@@ -1,15 +1,35 @@
-"""The 64x64 GEMM build's 128-k steps and the split layout's whole-block loads:
-first, odd and last steps and ragged tiles on the kernel emulator."""
+"""The GEMM's tile rules away from the 1024-pixel shapes, and the 64x64 build's
+128-k steps: the planned grids (no workgroup runs), the build's first, odd
+and last steps on the kernel emulator, and on the GPU the planned shapes
+against the oracle on sampled rows (2e-3 x RMS, the bar of fp16 operands),
+the unsplit ones bit for bit against another tile build.
+"""
 from __future__ import annotations
 
 import json
 
+import numpy as np
+import pytest
+
 from test_kemu import BOTH, _run, emulator  # noqa: F401  (fixture)
 
+ROUTES = [
+    ["gemm", [576, 1280, 1280], [180, 1, 1], 256], ["gemm_ws", [576, 1280, 1280], [180, 1, 1], 256],
+    ["gemm", [1600, 1280, 1280], [500, 1, 1], 256], ["gemm", [1976, 1280, 1280], [160, 1, 1], 512],
+    ["gemm", [3952, 640, 640], [155, 1, 1], 512], ["gemm", [7904, 640, 2560], [155, 1, 1], 512],
+    ["gemm_ws", [576, 1280, 5120], [50, 5, 1], 512], ["gemm_ws", [988, 1280, 5120], [80, 3, 1], 512],
+    ["gemm_ws", [1152, 1280, 5120], [50, 5, 1], 512], ["gemm_ws", [1024, 640, 2560], [160, 1, 1], 256],
+    ["gemm_ws", [4608, 640, 2560], [180, 1, 1], 512], ["gemm_ws", [308, 640, 2048], [50, 4, 1], 256],
+]
 EMULATED = [dict(M=70, N=70, K=128, cfg="3"), dict(M=65, N=130, K=384, layout="split", front=True, mode=1),
             dict(M=70, N=66, K=640, cfg="3:2"), dict(M=64, N=64, K=192, cfg="3", layout="split"),
             dict(M=200, N=140, K=192, cfg="6", layout="split", front=True), dict(case="gemm_geglu", M=70, F=40, K=384),
             dict(case="gemm_f16a", M=70, N=66, K=384)]
+
+
+def test_plans(emulator):  # noqa: F811
+    r = _run({"case": "routing", "table": ROUTES})
+    assert r.returncode == 0 and "OK routing" in r.stdout, (r.stdout + r.stderr)[-2000:]
 
 
 def test_steps_on_emulator(emulator):  # noqa: F811
@@ -21,3 +41,27 @@ def test_steps_on_emulator(emulator):  # noqa: F811
     bad = [f"{json.dumps(s)}\n{(r.stdout + r.stderr)[-800:]}" for s, r in zip(specs, results)
            if r.returncode != 0 or r.stdout.count("OK ") != len(BOTH)]
     assert not bad, "\n\n".join(bad)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,split", [(576, 1280, 5120, True), (988, 1280, 5120, True), (1152, 1280, 5120, True),
+                                         (1152, 1280, 1280, False), (3952, 640, 640, False), (7904, 640, 2560, False)])
+def test_planned_shapes(gpu, oracle, tune, M, N, K, split):
+    from helpers import REL_RMS_TOL, err_vs_rms, q8_weights
+    from sdvk_amd import ops
+    from sdvk_amd.hip import DeviceBuffer, synchronize
+
+    A, blocks = oracle.normal(1, M * K), q8_weights(oracle, 2, N, K)
+    dA, dW, dC = DeviceBuffer.from_array(A), DeviceBuffer.from_array(blocks), DeviceBuffer(M * N * 4)
+    nws = ops.gemm_workspace_bytes(M, N, K)
+    assert (nws > 0) == split
+    ops.gemm_nt_q8_0(dA, dW, dC, M, N, K, workspace=DeviceBuffer(nws) if nws else None)
+    synchronize()
+    got = dC.download(np.float32, M * N).reshape(M, N)
+    rows = np.unique(np.concatenate([[0, M - 1], np.random.default_rng(M).integers(0, M, 48)]))
+    assert err_vs_rms(got[rows], oracle.gemm_rows(A, blocks, M, N, K, rows, threads=oracle.max_threads())) <= REL_RMS_TOL
+    if not split:
+        tune("gemm_cfg", "5")
+        ops.gemm_nt_q8_0(dA, dW, dC, M, N, K)
+        synchronize()
+        assert np.array_equal(dC.download(np.float32, M * N).reshape(M, N), got)
