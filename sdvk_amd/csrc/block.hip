@@ -151,17 +151,15 @@ uint64_t ctx_kv_bytes(const mi_block_dims& d) {
     return 2 * round256(static_cast<uint64_t>(d.batch) * d.ctx_tokens * d.channels * (fp16_attention(d) ? 2 : 4));
 }
 
-// K and V of the context, into k / v (fp32, or fp16 with MI_BLOCK_FP16_ATTENTION).
-int ctx_kv(const mi_block_weights& w, const mi_block_dims& d, const float* ctx, void* k, void* v, hipStream_t s) {
-    const uint32_t crow = d.batch * d.ctx_tokens;
-    if (fp16_attention(d)) {
-        MI_TRY(mi_gemm_nt_q8_0_f16o(ctx, MI_F32, w.attn2_k, nullptr, k, crow, d.channels, d.ctx_channels, 0, 0, s));
-        return mi_gemm_nt_q8_0_f16o(ctx, MI_F32, w.attn2_v, nullptr, v, crow, d.channels, d.ctx_channels, 0, 0, s);
-    }
-    MI_TRY(mi_gemm_nt_q8_0(ctx, w.attn2_k, nullptr, static_cast<float*>(k), crow, d.channels, d.ctx_channels, 0, 0, 0,
-                           1, 0, 0, s));
-    return mi_gemm_nt_q8_0(ctx, w.attn2_v, nullptr, static_cast<float*>(v), crow, d.channels, d.ctx_channels, 0, 0, 0,
-                           1, 0, 0, s);
+// K and V of the context, into k / v (fp32, or fp16 with MI_BLOCK_FP16_ATTENTION), in
+// one launch: a 154-row projection alone fills 30 to 60 of the 256 CUs
+// (2 x 154x640x2048 31 -> 16 us).
+int ctx_kv(const mi_block_weights& w, const mi_block_dims& d, const float* ctx, void* k, void* v, hipStream_t s,
+           const char* fn) {
+    const void* W[2] = {w.attn2_k, w.attn2_v};
+    void* C[2] = {k, v};
+    return gemm_q8_0_shared_a(fn, ctx, false, W, C, 2, fp16_attention(d), d.batch * d.ctx_tokens, d.channels,
+                              d.ctx_channels, s);
 }
 
 // One block. Cross-attention K / V come from `kv` (K then V, ctx_kv_bytes
@@ -220,9 +218,10 @@ int forward(const mi_block_weights& w, const mi_block_dims& d, float* x, const f
         MI_TRY(proj(ws.n, w.attn1_q, ws.h, 3 * C));
         MI_TRY(attention(d, ws.h, at(ws.h, C), at(ws.h, 2ull * C), 3ull * C, ws.o, d.tokens, nullptr, hattn, half, s));
     } else {
-        MI_TRY(proj(ws.n, w.attn1_q, ws.q, C));
-        MI_TRY(proj(ws.n, w.attn1_k, ws.k, C));
-        MI_TRY(proj(ws.n, w.attn1_v, ws.v, C));
+        // one launch for the three (8192x640x640, 160 workgroups each: 3 x 18.8 -> 40 us)
+        const void* W[3] = {w.attn1_q, w.attn1_k, w.attn1_v};
+        void* qkv[3] = {ws.q, ws.k, ws.v};
+        MI_TRY(gemm_q8_0_shared_a(fn, ws.n, half, W, qkv, 3, hattn, rows, C, C, s));
         MI_TRY(attention(d, ws.q, ws.k, ws.v, C, ws.o, d.tokens, nullptr, hattn, half, s));
     }
     MI_TRY(residual(ws.o, w.attn1_out, w.attn1_out_b, C));
@@ -234,7 +233,7 @@ int forward(const mi_block_weights& w, const mi_block_dims& d, float* x, const f
         ck = kv;
         cv = static_cast<const char*>(kv) + ctx_kv_bytes(d) / 2;
     } else {
-        MI_TRY(ctx_kv(w, d, ctx, ws.k, ws.v, s));
+        MI_TRY(ctx_kv(w, d, ctx, ws.k, ws.v, s, fn));
     }
     MI_TRY(attention(d, ws.q, ck, cv, C, ws.o, d.ctx_tokens, ctx_len, hattn, half, s));
     MI_TRY(residual(ws.o, w.attn2_out, w.attn2_out_b, C));
@@ -284,7 +283,7 @@ extern "C" int mi_block_ctx_kv(const mi_block_weights* wt, const mi_block_dims* 
                     static_cast<unsigned long long>(kv_bytes), static_cast<unsigned long long>(ctx_kv_bytes(*dims)));
     if (!aligned(kv, 256)) return fail(MI_ERR_ALIGNMENT, "%s: kv buffer must be 256-byte aligned", fn);
     return ctx_kv(*wt, *dims, ctx, kv, reinterpret_cast<char*>(kv) + ctx_kv_bytes(*dims) / 2,
-                  static_cast<hipStream_t>(stream));
+                  static_cast<hipStream_t>(stream), fn);
 }
 
 extern "C" int mi_sdxl_block_forward_kv(const mi_block_weights* wt, const mi_block_dims* dims, float* x,

@@ -64,6 +64,14 @@ inline unsigned ceil_div(uint64_t a, uint64_t b) { return static_cast<unsigned>(
 void launch_splitk_reduce(const float* P, uint32_t splits, float* C, const float* bias, uint32_t M, uint32_t N,
                           uint32_t ldc, uint64_t sC, uint32_t batch, int op, hipStream_t s);
 
+// C[i] = A . deq(W[i])^T for `count` (at most three) Q8_0 weights of one [N, K] shape (34-byte blocks)
+// on the same A, in one launch: the matrices are grid z, so the grid fills the GPU
+// that one of them would leave partly idle. A [M, K] fp32 or fp16 (a_half), C[i] [M, N]
+// fp32 or fp16 (c_half: the fp32 result rounded once), all rows contiguous, C[i]
+// 16-byte aligned. The bits of `count` separate unsplit GEMMs (gemm_q8.hip).
+int gemm_q8_0_shared_a(const char* fn, const void* A, bool a_half, const void* const* W, void* const* C, uint32_t count,
+                       bool c_half, uint32_t M, uint32_t N, uint32_t K, hipStream_t s);
+
 // ----------------------------------------------------------- device helpers --
 
 // fp16 bit pattern -> fp32, exact for every pattern (subnormals scaled by

@@ -52,7 +52,22 @@ struct GemmArgs {
     uint32_t F;             // GEGLU epilogue: output columns (W has 2F rows: value rows, then gate rows)
     uint32_t out_half;      // GEGLU / plain mode-0 epilogue: output stored as fp16 (ldc in halves), the fp32 result rounded once
     uint64_t split_stride;  // K-split partials: elements between the planes of consecutive splits
+    // Bytes from W and C to those of grid z = 1 and 2: several weights on one A
+    // (gemm_q8_0_shared_a), else 0 and the batch strides. (Offsets, not pointers to
+    // choose from: those would make every C access a flat one.)
+    int64_t w1, w2, c1, c2;
 };
+
+// This workgroup's weights and output.
+__device__ __forceinline__ const uint8_t* weights_of(const GemmArgs& a) {
+    return a.W + (blockIdx.z == 1 ? a.w1 : blockIdx.z == 2 ? a.w2 : 0);
+}
+__device__ __forceinline__ float* output_of(const GemmArgs& a) {
+    const int64_t off = blockIdx.z == 1   ? a.c1
+                        : blockIdx.z == 2 ? a.c2
+                                          : static_cast<int64_t>(blockIdx.z) * static_cast<int64_t>(a.sC) * 4;
+    return reinterpret_cast<float*>(reinterpret_cast<char*>(a.C) + off);
+}
 
 // Epilogues. kEpiPlain: the reference's modes (0 stores acc + bias, 1 adds acc
 // to C). kEpiResidual: C += acc + bias (a residual add fused into the GEMM).
@@ -88,6 +103,8 @@ GemmArgs make_args(const float* A, const uint8_t* W, const float* scales, const 
     a.ldc = ldc;
     a.sA = sA;
     a.sC = sC;
+    a.c1 = static_cast<int64_t>(sC) * 4;
+    a.c2 = static_cast<int64_t>(sC) * 8;
     a.rowbytes = rowbytes;
     const uint32_t ldc_e = ldc ? ldc : N;
     a.cvec = (reinterpret_cast<uintptr_t>(C) % 16 == 0 && ldc_e % 4 == 0 && sC % 4 == 0) ? 1u : 0u;
@@ -455,8 +472,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     // 34-byte layout: records up to W's 16-byte-aligned end (the documented
     // read extent); the range check zeroes whole dwords only past that.
     const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(a.W), 0, static_cast<int>(WK == kBlocks34 ? (a.N * a.rowbytes + 15u) & ~15u : a.N * a.K),
-        0x00020000);
+        const_cast<uint8_t*>(weights_of(a)), 0,
+        static_cast<int>(WK == kBlocks34 ? (a.N * a.rowbytes + 15u) & ~15u : a.N * a.K), 0x00020000);
     const __amdgpu_buffer_rsrc_t rS =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(WK == kSplit ? a.scales : a.A), 0, -1, 0x00020000);
     uint32_t a_off[A_IT];
@@ -808,7 +825,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     }
     if (j < n_steps) compute(S0{});
 
-    float* C = a.C + static_cast<uint64_t>(blockIdx.z) * a.sC + (SPLITK ? blockIdx.y * a.split_stride : 0);
+    float* C = output_of(a) + (SPLITK ? blockIdx.y * a.split_stride : 0);
     __syncthreads();  // every wave is done with the operand tiles before LDS is reused
     const int wm_s = kFreshLane ? wave_s % WM : wm, wn_s = kFreshLane ? wave_s / WM : wn;
     store_tiles<FM, FN, SPLITK, EPI>(a, C, reinterpret_cast<float*>(smem) + wave_s * kStageFloats, m0 + wm_s * TM,
@@ -869,8 +886,8 @@ __global__ __launch_bounds__(512) void gemm_q8_rows_kernel(GemmArgs a) {
         const_cast<char*>(reinterpret_cast<const char*>(a.A) + static_cast<uint64_t>(blockIdx.z) * a.sA * AE), 0,
         static_cast<int>(((a.M - 1) * a.lda + a.K) * AE), 0x00020000);
     const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(a.W), 0, static_cast<int>(WK == kBlocks34 ? (a.N * a.rowbytes + 15u) & ~15u : a.N * a.K),
-        0x00020000);
+        const_cast<uint8_t*>(weights_of(a)), 0,
+        static_cast<int>(WK == kBlocks34 ? (a.N * a.rowbytes + 15u) & ~15u : a.N * a.K), 0x00020000);
     const __amdgpu_buffer_rsrc_t rS = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(WK == kSplit ? a.scales : a.A), 0, WK == kSplit ? static_cast<int>(a.N * nblk * 4) : 0,
         0x00020000);
@@ -968,10 +985,10 @@ __global__ __launch_bounds__(512) void gemm_q8_rows_kernel(GemmArgs a) {
     if (a.out_half) {
         // one RNE rounding of the fp32 value (as in store_tiles)
         asm volatile("" : "+v"(v));
-        reinterpret_cast<_Float16*>(a.C)[static_cast<uint64_t>(m) * a.ldc + out] = static_cast<_Float16>(v);
+        reinterpret_cast<_Float16*>(output_of(a))[static_cast<uint64_t>(m) * a.ldc + out] = static_cast<_Float16>(v);
         return;
     }
-    float* cp = a.C + static_cast<uint64_t>(blockIdx.z) * a.sC + static_cast<uint64_t>(m) * a.ldc + out;
+    float* cp = output_of(a) + static_cast<uint64_t>(m) * a.ldc + out;
     if (EPI == kEpiResidual || (EPI == kEpiPlain && a.mode != 0)) *cp += v;
     else *cp = v;
 }
@@ -1166,6 +1183,8 @@ GemmArgs partial_args(const GemmArgs& a, uint32_t splits, float* ws) {
     p.ldc = a.N;
     p.split_stride = static_cast<uint64_t>(a.M) * a.N;
     p.sC = p.split_stride * splits;
+    p.c1 = static_cast<int64_t>(p.sC) * 4;
+    p.c2 = static_cast<int64_t>(p.sC) * 8;
     return p;
 }
 
@@ -1748,6 +1767,43 @@ int gemm_f16out(const char* fn, const void* A, bool a_half, const void* W, const
     return check_launch(fn);
 }
 }  // namespace
+}  // namespace mi
+
+namespace mi {
+
+int gemm_q8_0_shared_a(const char* fn, const void* A, bool a_half, const void* const* W, void* const* C, uint32_t count,
+                       bool c_half, uint32_t M, uint32_t N, uint32_t K, hipStream_t stream) {
+    uint32_t mode = 0, lda = 0, ldc = 0;
+    const uint64_t wbytes = static_cast<uint64_t>(N) * (K / 32) * 34;
+    const uint64_t abytes = static_cast<uint64_t>(M) * K * (a_half ? 2 : 4), cbytes = static_cast<uint64_t>(M) * N * (c_half ? 2 : 4);
+    if (count == 0 || count > 3) return fail(MI_ERR_INVALID_ARG, "%s: %u weights", fn, count);
+    if (wbytes + 16 >= (uint64_t(1) << 32)) return fail(MI_ERR_UNSUPPORTED, "%s: weight >= 4 GiB", fn);
+    for (uint32_t i = 0; i < count; ++i) {
+        const int st = validate(fn, A, W[i], C[i], M, N, K, mode, lda, ldc, 1, 0, 0, true, a_half);
+        if (st) return st;
+        if (!aligned(W[i], 16)) return fail(MI_ERR_ALIGNMENT, "%s: W must be 16-byte aligned", fn);
+        if (!aligned(C[i], 16)) return fail(MI_ERR_ALIGNMENT, "%s: C must be 16-byte aligned", fn);
+        if (overlaps(C[i], cbytes, A, abytes) || overlaps(C[i], cbytes, W[i], wbytes))
+            return fail(MI_ERR_ALIASING, "%s: C overlaps an input", fn);
+    }
+    GemmArgs a = make_args(static_cast<const float*>(A), static_cast<const uint8_t*>(W[0]), nullptr, nullptr,
+                           static_cast<float*>(C[0]), M, N, K, 0, lda, ldc, 0, 0, (K / 32) * 34);
+    a.out_half = c_half ? 1u : 0u;
+    auto from = [](const void* x, const void* base) { return static_cast<const char*>(x) - static_cast<const char*>(base); };
+    if (count > 1) {
+        a.w1 = from(W[1], W[0]);
+        a.c1 = from(C[1], C[0]);
+    }
+    if (count > 2) {
+        a.w2 = from(W[2], W[0]);
+        a.c2 = from(C[2], C[0]);
+    }
+    const Plan p = choose(M, N, K, count, false);
+    if (a_half) dispatch<kBlocks34, kEpiPlain, true>(a, count, p, nullptr, stream);
+    else dispatch<kBlocks34, kEpiPlain>(a, count, p, nullptr, stream);
+    return check_launch(fn);
+}
+
 }  // namespace mi
 
 extern "C" int mi_gemm_nt_q8_0_f16o(const void* A, uint32_t a_dtype, const void* W, const float* bias, void* C,
