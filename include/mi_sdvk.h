@@ -389,18 +389,21 @@ int mi_add_inplace(float* x, const float* a, uint64_t n, void* stream);
  * or NULL. workspace: device memory of mi_block_workspace_bytes() bytes,
  * 256-byte aligned; nothing is allocated. Calls sharing a workspace must be
  * ordered (same stream).
- * dims.flags (0 = the reference's sequence of separate operators):
- *   MI_BLOCK_FUSED_EPILOGUES: the residual adds run in the out-projection /
- *     FF-down GEMM epilogues (mode 2) and GEGLU in the FF-up epilogue;
+ * Whatever the flags, the residual adds run in the out-projection / FF-down
+ * GEMM epilogues (mode 2), GEGLU in the FF-up epilogue, the separate Q / K / V
+ * projections in one launch, and -- where x and the LayerNorm parameters are
+ * 16-byte aligned -- the tensors whose only consumer is a GEMM (the LayerNorm,
+ * attention and GEGLU outputs) are stored as fp16 (each fp32 value rounded
+ * once, RNE, which is what the GEMM's A staging does to an fp32 tensor): the
+ * bits of the reference's sequence of separate operators on this library's
+ * entries. dims.flags:
+ *   MI_BLOCK_FUSED_EPILOGUES: accepted; always on;
+ *   MI_BLOCK_FP16_ACTIVATIONS: requires the fp16 hand-offs: an x or LayerNorm
+ *     parameter that is not 16-byte aligned is MI_ERR_ALIGNMENT;
  *   MI_BLOCK_JOINT_QKV: attn1_q / attn1_k / attn1_v are the three C x C parts
  *     of one [3C, C] Q8_0 matrix (attn1_k = attn1_q + C*(C/32)*34 bytes,
  *     attn1_v = attn1_k + as much; else MI_ERR_INVALID_ARG), projected by one
  *     GEMM;
- *   MI_BLOCK_FP16_ACTIVATIONS: the tensors whose only consumer is a GEMM --
- *     the LayerNorm outputs, the attention outputs and the GEGLU output --
- *     are stored as fp16 (each fp32 value rounded once, RNE, which is what the
- *     GEMM's A staging does to an fp32 tensor) and read by the fp16-A GEMM:
- *     half the bytes, no conversion in the GEMM;
  *   MI_BLOCK_FP16_ATTENTION: the Q / K / V projections and the cached
  *     context K / V are stored as fp16 (mi_gemm_nt_q8_0_f16o: the fp32 result
  *     rounded once) and both attentions take fp16 inputs, i.e. attention at the

@@ -414,8 +414,11 @@ __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
         for (int run = 0; run < 4; ++run) {
             const int d0 = 32 * u + 8 * run + 4 * g;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (d0 + e < hd) Op[d0 + e] = static_cast<TO>(o[u][4 * run + e] * inv);
+            for (int e = 0; e < 4; ++e) {
+                float v = o[u][4 * run + e] * inv;
+                asm volatile("" : "+v"(v));  // fp16 outputs: the fp32 product, rounded once more (half4_of)
+                if (d0 + e < hd) Op[d0 + e] = static_cast<TO>(v);
+            }
         }
 }
 

@@ -11,16 +11,25 @@
 // in a caller-provided workspace (nothing is allocated), every launch is
 // ordered on the caller's stream.
 //
+// What runs, whatever the flags (each of these computes the bits of the separate
+// operators):
+//   * the residual adds and biases in the epilogues of the out-projections and
+//     FF-down (GEMM mode 2), GEGLU in FF-up's epilogue (mi_gemm_nt_q8_0_geglu): no
+//     add passes, no [rows, 2 ff_inner] intermediate;
+//   * LayerNorm, attention and GEGLU outputs stored as fp16 for the GEMMs that read
+//     them (the GEMM rounds its A operand to fp16 anyway), where x and the LayerNorm
+//     parameters have the alignment of mi_layernorm_f16;
+//   * Q, K and V of self-attention, and K and V of the context, in one launch.
+// Against separate operators (Q / K / V in one launch already), MI355X, us per block with
+// fp32 attention: 2x4096x640 645 -> 538, 2x988x1280 358 -> 293, 2x576x1280 243 -> 203.
+//
 // mi_block_dims.flags:
-//   MI_BLOCK_FUSED_EPILOGUES: the out-projections and FF-down add their product
-//     and bias straight into x (GEMM mode 2) and FF-up applies GEGLU in its
-//     epilogue (mi_gemm_nt_q8_0_geglu), which removes the three residual-add
-//     passes and the [rows, 2 ff_inner] intermediate;
+//   MI_BLOCK_FUSED_EPILOGUES: accepted, always on;
+//   MI_BLOCK_FP16_ACTIVATIONS: the fp16 hand-offs are required: an x or LayerNorm
+//     parameter that is not 16-byte aligned is an error instead of taking fp32 ones;
 //   MI_BLOCK_JOINT_QKV: attn1 to_q / to_k / to_v are one [3C, C] Q8_0 matrix
-//     (the three pointers must be C x C matrices apart), projected by one GEMM;
-//   MI_BLOCK_FP16_ACTIVATIONS: LayerNorm, attention and GEGLU outputs stored as
-//     fp16 for the GEMMs that read them (the GEMM rounds its A operand to fp16
-//     anyway: the same bits);
+//     (the three pointers must be C x C matrices apart), projected by one GEMM with
+//     N = 3C (2-3% of the block faster than three matrices in one launch);
 //   MI_BLOCK_FP16_ATTENTION: the Q / K / V projections (and the cached context
 //     K / V) are stored as fp16, the RNE rounding of their fp32 results, and
 //     both attentions run on fp16 inputs (the fp16 kernel's pipeline) instead
@@ -28,17 +37,15 @@
 //     the precision of the library's fp16 attention entries; the block's bits
 //     differ from the flag-off block by that rounding.
 // Within one setting of MI_BLOCK_FP16_ATTENTION every variant computes the same bits: the GEMMs whose results must agree
-// across variants (Q / K / V, context K / V, FF-up) never split K, the
-// residual GEMMs split K the same way in both epilogue forms (partials in the
-// workspace, summed in a fixed order), and an unsplit GEMM's sums do not
-// depend on the tile build.
+// across variants (Q / K / V, context K / V, FF-up) never split K across
+// workgroups, and an unsplit GEMM's sums do not depend on the tile build.
 #include "common.hpp"
 
 namespace mi {
 namespace {
 
 struct Workspace {
-    float *n, *q, *k, *v, *o, *a, *h, *g;
+    float *n, *q, *k, *v, *o, *h, *g;
     float* split;           // K-split partials of the residual GEMMs
     uint64_t split_bytes;
 };
@@ -54,19 +61,17 @@ uint64_t split_bytes(const mi_block_dims& d) {
     return a > b ? a : b;
 }
 
-// Byte layout of the workspace; returns the total. h holds FF-up's
-// [rows, 2 ff_inner] output and, before the FF stage, the joint Q/K/V
+// Byte layout of the workspace; returns the total. h holds the joint Q/K/V
 // projection's [rows, 3C].
 uint64_t layout(const mi_block_dims& d, char* base, Workspace* w) {
     const uint64_t rows = static_cast<uint64_t>(d.batch) * d.tokens;
     const uint64_t crow = static_cast<uint64_t>(d.batch) * d.ctx_tokens;
     const uint64_t kvrows = rows > crow ? rows : crow;
-    const uint64_t hcols = 2ull * d.ff_inner > 3ull * d.channels ? 2ull * d.ff_inner : 3ull * d.channels;
-    const uint64_t sizes[8] = {rows * d.channels, rows * d.channels, kvrows * d.channels, kvrows * d.channels,
-                               rows * d.channels, rows * d.channels, rows * hcols, rows * d.ff_inner};
-    float** slots[8] = {&w->n, &w->q, &w->k, &w->v, &w->o, &w->a, &w->h, &w->g};
+    const uint64_t sizes[7] = {rows * d.channels, rows * d.channels, kvrows * d.channels, kvrows * d.channels,
+                               rows * d.channels, rows * 3ull * d.channels, rows * d.ff_inner};
+    float** slots[7] = {&w->n, &w->q, &w->k, &w->v, &w->o, &w->h, &w->g};
     uint64_t off = 0;
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < 7; ++i) {
         if (base) *slots[i] = reinterpret_cast<float*>(base + off);
         off += round256(sizes[i] * 4);
     }
@@ -162,6 +167,14 @@ int ctx_kv(const mi_block_weights& w, const mi_block_dims& d, const float* ctx, 
                               d.ctx_channels, s);
 }
 
+// mi_layernorm_f16 serves the block's LayerNorms.
+bool half_handoffs(const mi_block_weights& w, const mi_block_dims& d, const float* x) {
+    const float* p[6] = {w.norm1_w, w.norm1_b, w.norm2_w, w.norm2_b, w.norm3_w, w.norm3_b};
+    for (const float* q : p)
+        if (!aligned(q, 16)) return false;
+    return aligned(x, 16) && d.channels <= kLayerNormVecMax;
+}
+
 // One block. Cross-attention K / V come from `kv` (K then V, ctx_kv_bytes
 // layout) when given, else are projected from `ctx` into the workspace.
 int forward(const mi_block_weights& w, const mi_block_dims& d, float* x, const float* ctx, const void* kv,
@@ -176,20 +189,12 @@ int forward(const mi_block_weights& w, const mi_block_dims& d, float* x, const f
     if (!aligned(workspace, 256)) return fail(MI_ERR_ALIGNMENT, "%s: workspace must be 256-byte aligned", fn);
 
     const uint32_t rows = d.batch * d.tokens, C = d.channels;
-    const uint64_t nx = static_cast<uint64_t>(rows) * C;
-    const bool fused = (d.flags & MI_BLOCK_FUSED_EPILOGUES) != 0;
-    // fp16 activations: n (LayerNorm out), o (attention out) and g (GEGLU out)
-    // hold fp16 and feed the fp16-A GEMM (same bits as fp32 + staging)
-    const bool half = (d.flags & MI_BLOCK_FP16_ACTIVATIONS) != 0;
+    // n (LayerNorm out), o (attention out) and g (GEGLU out) hold fp16 and feed the
+    // fp16-A GEMM: the bits of fp32 hand-offs, half the bytes
+    const bool half = (d.flags & MI_BLOCK_FP16_ACTIVATIONS) != 0 || half_handoffs(w, d, x);
     auto gemm = [&](const void* A, const void* W, const float* bias, float* out, uint32_t M, uint32_t N, uint32_t K) {
         if (half) return mi_gemm_nt_q8_0_f16a(A, W, bias, out, M, N, K, 0, 0, 0, 1, 0, 0, nullptr, 0, s);
         return mi_gemm_nt_q8_0(static_cast<const float*>(A), W, bias, out, M, N, K, 0, 0, 0, 1, 0, 0, s);
-    };
-    auto gemm_ws = [&](const void* A, const void* W, const float* bias, float* out, uint32_t K, uint32_t mode) {
-        if (half) return mi_gemm_nt_q8_0_f16a(A, W, bias, out, rows, C, K, mode, 0, 0, 1, 0, 0, ws.split,
-                                              ws.split_bytes, s);
-        return mi_gemm_nt_q8_0_ws(static_cast<const float*>(A), W, bias, out, rows, C, K, mode, 0, 0, 1, 0, 0,
-                                  ws.split, ws.split_bytes, s);
     };
     // MI_BLOCK_FP16_ATTENTION: the Q / K / V projections store fp16 (element
     // offsets below count halves then)
@@ -203,17 +208,15 @@ int forward(const mi_block_weights& w, const mi_block_dims& d, float* x, const f
     auto layernorm = [&](const float* g, const float* b) {
         return half ? mi_layernorm_f16(x, g, b, ws.n, rows, C, 1e-5f, s) : mi_layernorm(x, g, b, ws.n, rows, C, 1e-5f, s);
     };
-    // x += A . W^T + bias: one GEMM with the residual epilogue, or GEMM + add;
-    // both split K the same way (the workspace's partials region)
+    // x += A . W^T + bias
     auto residual = [&](const void* A, const void* W, const float* bias, uint32_t K) {
-        if (fused) return gemm_ws(A, W, bias, x, K, 2);
-        const int st = gemm_ws(A, W, bias, ws.a, K, 0);
-        return st != MI_OK ? st : mi_add_inplace(x, ws.a, nx, s);
+        if (half) return mi_gemm_nt_q8_0_f16a(A, W, bias, x, rows, C, K, 2, 0, 0, 1, 0, 0, ws.split, ws.split_bytes, s);
+        return mi_gemm_nt_q8_0_ws(static_cast<const float*>(A), W, bias, x, rows, C, K, 2, 0, 0, 1, 0, 0, ws.split,
+                                  ws.split_bytes, s);
     };
 
     // self-attention
     MI_TRY(layernorm(w.norm1_w, w.norm1_b));
-    // the joint result [rows, 3C] goes to the FF-up region, free until the FF stage
     if (d.flags & MI_BLOCK_JOINT_QKV) {
         MI_TRY(proj(ws.n, w.attn1_q, ws.h, 3 * C));
         MI_TRY(attention(d, ws.h, at(ws.h, C), at(ws.h, 2ull * C), 3ull * C, ws.o, d.tokens, nullptr, hattn, half, s));
@@ -239,14 +242,8 @@ int forward(const mi_block_weights& w, const mi_block_dims& d, float* x, const f
     MI_TRY(residual(ws.o, w.attn2_out, w.attn2_out_b, C));
     // GEGLU feed-forward
     MI_TRY(layernorm(w.norm3_w, w.norm3_b));
-    if (fused) {
-        if (half) MI_TRY(mi_gemm_nt_q8_0_geglu_f16(ws.n, w.ff_up, w.ff_up_b, ws.g, rows, d.ff_inner, C, 0, 0, s));
-        else MI_TRY(mi_gemm_nt_q8_0_geglu(ws.n, w.ff_up, w.ff_up_b, ws.g, rows, d.ff_inner, C, 0, 0, s));
-    } else {
-        MI_TRY(gemm(ws.n, w.ff_up, w.ff_up_b, ws.h, rows, 2 * d.ff_inner, C));
-        if (half) MI_TRY(mi_geglu_f16(ws.h, ws.g, rows, d.ff_inner, s));
-        else MI_TRY(mi_geglu(ws.h, ws.g, rows, d.ff_inner, s));
-    }
+    if (half) MI_TRY(mi_gemm_nt_q8_0_geglu_f16(ws.n, w.ff_up, w.ff_up_b, ws.g, rows, d.ff_inner, C, 0, 0, s));
+    else MI_TRY(mi_gemm_nt_q8_0_geglu(ws.n, w.ff_up, w.ff_up_b, ws.g, rows, d.ff_inner, C, 0, 0, s));
     MI_TRY(residual(ws.g, w.ff_down, w.ff_down_b, d.ff_inner));
     return MI_OK;
 }

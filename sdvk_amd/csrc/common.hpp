@@ -72,6 +72,9 @@ void launch_splitk_reduce(const float* P, uint32_t splits, float* C, const float
 int gemm_q8_0_shared_a(const char* fn, const void* A, bool a_half, const void* const* W, void* const* C, uint32_t count,
                        bool c_half, uint32_t M, uint32_t N, uint32_t K, hipStream_t s);
 
+// The longest row of the vector LayerNorm (mi_layernorm_f16's limit; glue.hip).
+constexpr uint32_t kLayerNormVecMax = 4096;
+
 // ----------------------------------------------------------- device helpers --
 
 // fp16 bit pattern -> fp32, exact for every pattern (subnormals scaled by

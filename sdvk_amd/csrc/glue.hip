@@ -23,6 +23,7 @@ namespace mi {
 namespace {
 
 constexpr int kLnCache = 16;  // float4 per lane cached in registers: rows up to 64 * 4 * 16 = 4096
+static_assert(64 * 4 * kLnCache == kLayerNormVecMax, "the vector LayerNorm's longest row");
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
