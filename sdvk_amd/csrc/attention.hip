@@ -182,8 +182,8 @@ constexpr float kLazy = 8.0f;
 constexpr float kLazySum = 256.0f;
 
 // Tensors whose rows are not 16-byte aligned, or with a head dim that is not a
-// multiple of 8: element-wise loads and stores (VEC = false, the only build: the
-// others take the pipelined kernels below).
+// multiple of 8, and fp32 grids past a 1-D launch: element-wise loads and stores
+// (VEC = false, the only build: the others take the pipelined kernels below).
 template <typename TI, typename TO, bool VEC>
 __global__ __launch_bounds__(kThreads) void attn_kernel(AttnArgs a) {
     static_assert(!VEC, "16-byte aligned tensors take the pipelined kernels");
@@ -1627,9 +1627,12 @@ int run(const mi_attn_args& x, hipStream_t s, const char* fn, void* ws = nullptr
                      (so * eo) % vout == 0 && (a.hd * ei) % vin == 0;
     // fp16 inputs on the vector path: the pipelined kernel (one workgroup per
     // 64 or 128 queries of one (batch, head), 1-D grid)
-    const bool small_grid = static_cast<uint64_t>(ceil_div(x.Tq, 64u)) * x.heads * x.batch < (1ull << 31);
-    const bool fast = vec && x.in_dtype == MI_F16 && small_grid;
-    const bool fast32 = vec && x.in_dtype == MI_F32 && small_grid;
+    const bool fast = vec && x.in_dtype == MI_F16 &&
+                      static_cast<uint64_t>(ceil_div(x.Tq, 64u)) * x.heads * x.batch < (1ull << 31);
+    // fp32 inputs likewise: a 1-D grid of 512-thread workgroups, and a launch takes fewer
+    // than 2^32 threads a dimension (larger grids keep the 3-D one of attn_kernel)
+    const bool fast32 = vec && x.in_dtype == MI_F32 &&
+                        static_cast<uint64_t>(ceil_div(x.Tq, kBQ)) * x.heads * x.batch < (1ull << 23);
     a.nfull = 0;
     a.pieces = 1;
     a.part = nullptr;

@@ -75,3 +75,20 @@ def test_on_gpu(gpu, oracle, B, Tq, Tk, C, heads, causal, pad, scale):
         e = np.abs(got[:, :, :C] - want) / (bar + (2.0 ** -11 * (spread + np.abs(want)) if precision else 0.0))
         print(f"[case] {B}x{heads}x{Tq}x{Tk} precision {precision}: {e.max():.2f} of the bar", flush=True)
         assert e.max() <= 1.0
+
+
+@pytest.mark.gpu
+def test_more_workgroups_than_a_1d_launch(gpu):
+    """2^24 and more (batch, head) pairs: 256 threads each no longer fit one grid dimension. One key: out = v."""
+    from sdvk_amd import MI_F32, ops
+    from sdvk_amd.hip import DeviceBuffer, synchronize
+
+    B, heads, hd = 65535, 257, 8
+    v = np.arange(B * heads * hd, dtype=np.float32) % 8191
+    dv = DeviceBuffer.from_array(v)
+    dq, do = DeviceBuffer.from_array(np.ones_like(v)), DeviceBuffer(v.nbytes)
+    ops.fused_attention_ex(dq, dq, dv, do, batch=B, Tq=1, Tk=1, C=heads * hd, heads=heads, in_dtype=MI_F32,
+                           out_dtype=MI_F32)
+    synchronize()
+    # values below 2^13 are whole: one key's weight is 1, hi + lo carries 2^-22 of a value
+    assert np.abs(do.download(np.float32, v.size) - v).max() <= 8191 * 2.0 ** -21
