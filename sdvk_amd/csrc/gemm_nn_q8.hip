@@ -52,7 +52,8 @@ struct NnArgs {
     uint32_t M, N, K, mode, lda, ldb, ldc;
     uint32_t sA, sB, sC;                      // batch strides (elements), < 2^31 by validation
     uint32_t a_bytes, s_bytes, b_bytes, c_bytes;  // whole-buffer extents
-    uint32_t splits, steps_per_split;         // tiled kernel: K splits (blockIdx.z = batch * splits + split)
+    uint32_t splits, steps_per_split;         // tiled kernel: K splits (grid z = batch * splits + split)
+    uint32_t by_xcd;                          // tiled kernel: tiles handed out by XCD (nn_by_xcd)
     uint64_t plane;                           // K splits: floats per partial plane (C = workspace, ldc = N)
 };
 
@@ -159,14 +160,24 @@ __global__ __launch_bounds__(kNT2) void gemm_nn_q8_tiled_kernel(NnArgs a) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, g = lane >> 5;
     const int wm = wave & 1, wn = wave >> 1;
-    const uint32_t n0 = blockIdx.x * kBN2, m0 = blockIdx.y * kBM2;
+    // This workgroup's tile (nn_by_xcd): the grid's own order, or a run of tiles per XCD
+    // with the rows of C fastest, so that the workgroups that share B share an L2.
+    uint32_t tn = blockIdx.x, tm = blockIdx.y, zs = blockIdx.z;
+    if (a.by_xcd) {
+        const uint32_t t = xcd_swizzle(tn + gridDim.x * (tm + gridDim.y * zs), gridDim.x * gridDim.y * gridDim.z);
+        const uint32_t q = t / gridDim.y;
+        tm = t - q * gridDim.y;
+        zs = q / gridDim.x;
+        tn = q - zs * gridDim.x;
+    }
+    const uint32_t n0 = tn * kBN2, m0 = tm * kBM2;
     // B in LDS: row n holds its 64 k as 16 units of 4 halves, unit u at slot
     // u ^ 2 ((n / 16) % 4). The 8-byte writes of the store phase (32 lanes:
     // 16 quads of n x 2 k blocks) then cover all 64 banks once, and the 16-byte
     // fragment reads (16 consecutive rows, one even unit pair) stay
     // conflict-free and 16-byte aligned.
     auto b_slot = [](uint32_t n, uint32_t u) { return n * kLd2 + 4 * (u ^ (2 * ((n >> 4) & 3))); };
-    const uint32_t z = blockIdx.z / a.splits, split = blockIdx.z % a.splits;
+    const uint32_t z = zs / a.splits, split = zs % a.splits;
     const uint32_t ksteps = a.K / kBK2;
     const uint32_t s_begin = SPLITK ? split * a.steps_per_split : 0;
     const uint32_t s_end = SPLITK ? min(ksteps, s_begin + a.steps_per_split) : ksteps;
@@ -350,6 +361,19 @@ uint32_t nn_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t batch) {
     return splits;
 }
 
+// Whether the tiled kernel hands its tiles out by XCD. Workgroup i of a launch runs on
+// XCD i % 8, so with a multiple of four column tiles a column of B (all its row tiles
+// and K splits) stays on one or two XCDs by itself; with any other number the row
+// tiles that read the same B sit on up to eight, and each of their L2s fetches it. Below
+// 2 MB (half an XCD's L2) every L2 keeps all of B in either order. Measured on MI355X,
+// us, grid order / by XCD: 640x1600x5760 (7 column tiles) 45.7 / 31.5, 640x2304x5760 (9)
+// 55.1 / 43.6, 640x3456x5760 (14) 68.4 / 63.3, 1280x576x11520 (3) 48.9 / 42.1,
+// 1280x256x11520 (1) 33.3 / 27.8; the other way round 1280x1024x11520 (4) 63.8 / 65.5,
+// 640x4096x320 (16) 12.0 / 12.2, 1280x576x640 (3, 1.5 MB) 14.8 / 15.0.
+bool nn_by_xcd(uint32_t N, uint32_t K) {
+    return ceil_div(N, kBN2) % 4 != 0 && static_cast<uint64_t>(K) * N * 4 > (2u << 20);
+}
+
 int gemm_nn(const char* fn, const uint32_t* payload, const float* scales, const float* B, float* C, uint32_t M,
             uint32_t N, uint32_t K, uint32_t mode, uint32_t lda, uint32_t ldb, uint32_t ldc, uint32_t batch,
             uint64_t sA, uint64_t sB, uint64_t sC, void* ws, uint64_t ws_bytes, hipStream_t st) {
@@ -415,6 +439,7 @@ int gemm_nn(const char* fn, const uint32_t* payload, const float* scales, const 
         gemm_nn_q8_kernel<<<grid, 256, 0, st>>>(a);
         return check_launch(fn);
     }
+    a.by_xcd = nn_by_xcd(N, K) ? 1u : 0u;
     const uint32_t ksteps = K / kBK2;
     uint32_t splits = ws ? nn_splits(M, N, K, batch) : 1;
     const uint64_t plane = static_cast<uint64_t>(M) * N;
