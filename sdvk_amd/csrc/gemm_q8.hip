@@ -386,6 +386,9 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& a, float* C, float* 
 template <int BM, int BN, int WM, int WN, int KB, int WK, bool SPLITK, bool KTAIL, int PF, int EPI = kEpiPlain,
           bool AH = false, bool PP = false>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
+    // several weights on one A (gemm_q8_0_shared_a); selecting them by grid z in every build cost
+    // the K-split and GEGLU ones up to 1% (154x1280x2048 9.96 against 9.89 us, 1976x5120x1280 70.7 / 69.9)
+    constexpr bool kShared = EPI == kEpiPlain && !SPLITK;
     constexpr int NT = WM * WN * 64;
     constexpr int BK = 32 * KB;
     constexpr int LDK = BK + 8;                   // LDS row stride in halves (16-B pad)
@@ -472,7 +475,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     // 34-byte layout: records up to W's 16-byte-aligned end (the documented
     // read extent); the range check zeroes whole dwords only past that.
     const __amdgpu_buffer_rsrc_t rW = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(weights_of(a)), 0,
+        const_cast<uint8_t*>(kShared ? weights_of(a) : a.W), 0,
         static_cast<int>(WK == kBlocks34 ? (a.N * a.rowbytes + 15u) & ~15u : a.N * a.K), 0x00020000);
     const __amdgpu_buffer_rsrc_t rS =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(WK == kSplit ? a.scales : a.A), 0, -1, 0x00020000);
@@ -825,7 +828,8 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     }
     if (j < n_steps) compute(S0{});
 
-    float* C = output_of(a) + (SPLITK ? blockIdx.y * a.split_stride : 0);
+    float* C = kShared ? output_of(a)
+                       : a.C + static_cast<uint64_t>(blockIdx.z) * a.sC + (SPLITK ? blockIdx.y * a.split_stride : 0);
     __syncthreads();  // every wave is done with the operand tiles before LDS is reused
     const int wm_s = kFreshLane ? wave_s % WM : wm, wn_s = kFreshLane ? wave_s / WM : wn;
     store_tiles<FM, FN, SPLITK, EPI>(a, C, reinterpret_cast<float*>(smem) + wave_s * kStageFloats, m0 + wm_s * TM,
