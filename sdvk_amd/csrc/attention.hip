@@ -439,9 +439,13 @@ constexpr int kResidNone = 0, kResidDiagonal = 1, kResidAll = 2;
 //     issues the score MFMAs of the next sub-tile between the exponentials and
 //     fp16 packing of this one; phase B issues this sub-tile's PV MFMAs between
 //     the conversion and LDS stores of the next tile;
-//   * the running max enters as the score MFMA's initial accumulator (-m, in raw
-//     score units, one register block that changes only when m does), so an
-//     exponential costs one multiply by scale * log2 e and the exp itself;
+//   * the running max m (exp2 domain) enters the fma that scales a score, so an
+//     exponential costs that fma and the exp itself. (As the score MFMA's initial
+//     accumulator, -m in raw units, it takes their low bits from the scores of a
+//     sub-tile far above m, before the rescale sees them: first keys 1000 below the
+//     rest gave errors of 2.3e-4 of the RMS where 1e-6 is due.) A score's eight
+//     MFMAs with a residual come first, so that only four round at its own size:
+//     1 x 10 x 2304^2 48.5 -> 48.2 us, error against 64 bits 4.7e-7 -> 4.5e-7;
 //   * as in the fp16 kernel no row max is taken per tile: the sum of a sub-tile's P
 //     bounds each of them, and a sum over 2^8 (rare) sends the wave through a
 //     rescale;
@@ -464,7 +468,7 @@ constexpr int kResidNone = 0, kResidDiagonal = 1, kResidAll = 2;
 //
 // What bounds it: MFMA and VALU issue, close together. Per wave, 64 keys and 32
 // queries: 24 score + 16 PV MFMAs (24 with P's residual) of 34 cycles, and 32
-// multiplies, 32 exponentials (8.5 cycles each), 32 packed conversions and 32 or 64
+// fmas, 32 exponentials (8.5 cycles each), 32 packed conversions and 32 or 64
 // mixed fmas (9 cycles each) on the VALU. Measured on MI355X against the unpipelined
 // kernel it replaces, us: mi_fused_attention 1 x 10 x 2304^2 77.3 -> 48.7 (280
 // TFLOP/s), 1 x 10 x 4096^2 219 -> 165, 2 x 10 x 4096^2 with fp16 P 290 -> 234, cross
@@ -572,9 +576,9 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
     };
 
     half8 qh[4], ql[4];
-    floatx16 o[2], mneg;
+    floatx16 o[2];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[0][r] = o[1][r] = mneg[r] = 0.0f;
+    for (int r = 0; r < 16; ++r) o[0][r] = o[1][r] = 0.0f;
     float lsum = 0.0f, m = 0.0f;
     const float c = fabsf(a.c);  // a negative scale is taken into Q
 
@@ -585,6 +589,13 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
         const _Float16* S = stage0 + st * kFStage + k_rd + 32 * t * kFLd + 16 * s4;
         kh[s4] = *reinterpret_cast<const half8*>(S);
         kl[s4] = *reinterpret_cast<const half8*>(S + kFPlane);
+    };
+    // The i-th of a sub-tile's 12 score MFMAs: the eight with a residual first, so that
+    // only the last four round at the size of the score.
+    auto score_mfma = [&](int i, const floatx16& s) {
+        const int s4 = i < 8 ? i / 2 : i - 8;
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(i < 8 && i % 2 ? kl[s4] : kh[s4], i < 8 && i % 2 == 0 ? ql[s4] : qh[s4],
+                                                      s, 0, 0, 0);
     };
     // V^T fragments of PV step (t, sp), columns 32u .. 32u + 31
     half8 vh[2][2], vl[2][2];
@@ -620,8 +631,8 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
     float ts;
     const half2 one2 = {1, 1};
     auto exps = [&](const floatx16& s, int i) {
-        p[2 * i] = __builtin_amdgcn_exp2f(s[2 * i] * c);
-        p[2 * i + 1] = __builtin_amdgcn_exp2f(s[2 * i + 1] * c);
+        p[2 * i] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i], c, -m));
+        p[2 * i + 1] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i + 1], c, -m));
     };
     auto soft = [&](const floatx16& s, int i) {  // the next pair's exponentials, then pack pair i
         if (i < 7) exps(s, i + 1);
@@ -638,21 +649,17 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
         const half2* y = x + 4 * sp;
         return half8{y[0][0], y[0][1], y[1][0], y[1][1], y[2][0], y[2][1], y[3][0], y[3][1]};
     };
-    // Adds the sub-tile's sum after the lazy-rescale test; next: the scores of
-    // the following sub-tile, already taken against the old m.
-    auto settle = [&](floatx16& s, floatx16& next) {
+    // Adds the sub-tile's sum after the lazy-rescale test.
+    auto settle = [&](const floatx16& s) {
         if (__any(ts > kLazySum)) {
-            const float d = fmaxf(lane_max(s), 0.0f);
-            const float alpha = __builtin_amdgcn_exp2f(-d * c);
-            m += d;
+            const float m_new = fmaxf(m, lane_max(s) * c);
+            const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+            m = m_new;
             lsum *= alpha;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 o[0][r] *= alpha;
                 o[1][r] *= alpha;
-                mneg[r] = -m;
-                s[r] -= d;
-                next[r] -= d;
             }
             ts = 0.0f;
             exps(s, 0);
@@ -661,7 +668,7 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
         }
         lsum += ts;
     };
-    // Phase A: next = scores of sub-tile (st, t) against m (12 MFMAs in a chain),
+    // Phase A: next = scores of sub-tile (st, t) (12 MFMAs in a chain),
     // P of s between them; the first V fragments of the PV phase (vst, vt) that
     // follows are read at its end. The scheduler's barriers hold each piece of
     // vector work behind its MFMA (left alone the compiler issues the MFMAs in a
@@ -669,19 +676,15 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
     auto phase_a = [&](const floatx16& s, floatx16& next, int st, int t, auto VNEXT, int vst, int vt) {
         ts = 0.0f;
         exps(s, 0);
-        next = mneg;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) next[r] = 0.0f;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-            if (s4 < 2) read_k(st, t, s4 + 2);
-            if (decltype(VNEXT)::value && s4 == 3) read_v(vst, vt, 0);
-            next = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[s4], qh[s4], next, 0, 0, 0);
-            soft(s, 2 * s4);
-            __builtin_amdgcn_sched_barrier(0);
-            next = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[s4], ql[s4], next, 0, 0, 0);
-            soft(s, 2 * s4 + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            next = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[s4], qh[s4], next, 0, 0, 0);
+        for (int i = 0; i < 12; ++i) {
+            if (i == 0 || i == 2) read_k(st, t, 2 + i / 2);
+            if (decltype(VNEXT)::value && i == 9) read_v(vst, vt, 0);
+            next = score_mfma(i, next);
+            if (i % 3 != 2) soft(s, i / 3 * 2 + i % 3);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -769,24 +772,18 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
         for (int i = 0; i < 4; ++i) store_unit(1, i);
         load_v(min(1u, n - 1));  // V before K, as in the loop (loads retire in issue order)
         load_k(min(2u, n - 1));
-        floatx16 s0 = mneg, s1;
+        floatx16 s0, s1;
 #pragma unroll
-        for (int s4 = 0; s4 < 4; ++s4) {
-            read_k(0, 0, s4);
-            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[s4], qh[s4], s0, 0, 0, 0);
-            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kh[s4], ql[s4], s0, 0, 0, 0);
-            s0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(kl[s4], qh[s4], s0, 0, 0, 0);
-        }
+        for (int r = 0; r < 16; ++r) s0[r] = 0.0f;
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4) read_k(0, 0, s4);
+#pragma unroll
+        for (int i = 0; i < 12; ++i) s0 = score_mfma(i, s0);
         if (grp * kBKV + 32 > kfull) mask(s0, grp * kBKV);
         // the first sub-tile's max (a group whose first sub-tile is masked for a
         // query has no key of that query at all: its keys only ascend)
         const float mx0 = lane_max(s0);
-        m = mx0 == -INFINITY ? 0.0f : mx0;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            mneg[r] = -m;
-            s0[r] -= m;
-        }
+        m = mx0 == -INFINITY ? 0.0f : mx0 * c;
         read_k(0, 1, 0);
         read_k(0, 1, 1);
         // At the top of trip j: K tiles j and j + 1 and V tile j staged (or being
@@ -797,7 +794,7 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
             const int st = j & 1;
             const uint32_t kv0 = (j * KG + grp) * kBKV;
             phase_a(s0, s1, st, 1, std::false_type{}, st, 0);
-            settle(s0, s1);
+            settle(s0);
             if (kv0 + 64 > kfull) mask(s1, kv0 + 32);
             // tile j's V and tile j + 1's K are whole; every wave is done with tile
             // j's K and tile j - 1's V
@@ -807,7 +804,7 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
             load_v(min(j + 2, n - 1));
             __builtin_amdgcn_sched_barrier(0);
             phase_a(s1, s0, st ^ 1, 0, std::true_type{}, st, 1);
-            settle(s1, s0);
+            settle(s1);
             if (kv0 + KG * kBKV + 32 > kfull) mask(s0, kv0 + KG * kBKV);
             __builtin_amdgcn_sched_barrier(0);
             phase_b(std::true_type{}, st, 1, st, 0, st ^ 1, 1);
@@ -838,8 +835,8 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
         const float l1 = ML[64 + lane];
         const float m0 = lt != 0.0f ? m : -INFINITY, m1 = l1 != 0.0f ? ML[lane] : -INFINITY;
         const float M = fmaxf(m0, m1);
-        const float a0 = m0 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m0 - M) * c);
-        const float a1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m1 - M) * c);
+        const float a0 = m0 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m0 - M);
+        const float a1 = m1 == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m1 - M);
         lt = a0 * lt + a1 * l1;
 #pragma unroll
         for (int u = 0; u < 2; ++u)

@@ -203,13 +203,15 @@ def gemm_nn(E, *, M, N, K, mode=0, batch=1, lda=0, ldb=0, ldc=0, sA=0, sB=0, sC=
 
 def attention(E, *, batch=1, Tq, Tk, C, heads, causal=False, f16_in=False, f16_out=False, kv_len=None, seed=1,
               front=False, order=0, tol=2e-3, nw=None, outliers=None, direct_store=False, split=None,
-              precise=False, precision=None, simd_waves=None):
+              precise=False, precision=None, simd_waves=None, low=None):
     """mi_fused_attention_ex (contiguous [batch, T, C]) against the oracle;
     split "<rest>:<pieces>": through mi_fused_attention_ws with that key-split
     plan forced (the attn_split override) and the workspace the library asks
     for; nw pins the fp16 kernel's workgroup size (attn_nw); outliers: key
     indices whose scores stand far above the rest (q ~ 1, k ~ 0.1 N(0, 1),
     those keys 3.0), so that a running max that misses them overflows;
+    low [n, d]: the scores of the first n keys stand d below the rest (one
+    feature of every head);
     direct_store: output stores straight from the MFMA layout
     (attn_direct_store) instead of whole rows through LDS; precision: the
     mi_attn_args field, by default MI_ATTN_PREC_FP16 (one fp16 P product);
@@ -232,6 +234,12 @@ def attention(E, *, batch=1, Tq, Tk, C, heads, causal=False, f16_in=False, f16_o
         kk = (k.astype(np.float32) * np.float32(0.1)).reshape(batch, Tk, C)
         kk[:, outliers, :] = 3.0
         k = kk.reshape(-1).astype(idt)
+    if low:
+        hd = C // heads
+        q.reshape(-1, hd)[:, 0] = 1.0
+        kk = k.reshape(batch, Tk, heads, hd)
+        kk[..., 0] = 0.0
+        kk[:, :low[0], :, 0] = -low[1] * np.sqrt(hd)
     odt = np.float16 if f16_out else np.float32
     n_out = batch * Tq * C
     dq, dk, dv = E.buf(q, front=front), E.buf(k, front=front), E.buf(v, front=front)

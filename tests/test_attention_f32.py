@@ -45,6 +45,42 @@ def test_on_emulator(emulator):  # noqa: F811
     assert not bad, "\n\n".join(bad)
 
 
+# First keys far below the rest, in one and two sub-tiles, one and two key groups: the scores
+# that follow are taken before the running max leaves its first value and must keep
+# fp32's bits, so the plain bar holds whatever the distance.
+LOW = [dict(Tq=40, Tk=96, C=64, heads=1, low=[32, 1000]), dict(Tq=33, Tk=200, C=128, heads=2, low=[40, 100]),
+       dict(Tq=40, Tk=600, C=64, heads=1, low=[32, 5000])]
+
+
+def test_low_first_keys_on_emulator(emulator):  # noqa: F811
+    from concurrent.futures import ThreadPoolExecutor
+
+    specs = [dict({"case": "attention"}, schedules=BOTH, precision=0, tol=2e-5, **s) for s in LOW]
+    with ThreadPoolExecutor(4) as ex:
+        results = list(ex.map(_run, specs))
+    bad = [f"{json.dumps(s)}\n{(r.stdout + r.stderr)[-800:]}" for s, r in zip(specs, results)
+           if r.returncode != 0 or r.stdout.count("OK ") != len(BOTH)]
+    assert not bad, "\n\n".join(bad)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Tk,n,d", [(96, 32, 1000.0), (200, 40, 100.0), (600, 32, 5000.0), (1024, 64, 300.0)])
+def test_low_first_keys_on_gpu(gpu, oracle, Tk, n, d):
+    from sdvk_amd import MI_F32, ops
+    from sdvk_amd.hip import DeviceBuffer, synchronize
+
+    q, k, v = (oracle.normal(i, t * 64).reshape(t, 64) for i, t in ((1, 130), (2, Tk), (3, Tk)))
+    q[:, 0], k[:, 0], k[:n, 0] = 1.0, 0.0, -8.0 * d
+    s = q.astype(np.float64) @ k.astype(np.float64).T / 8.0
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = p @ v.astype(np.float64) / p.sum(-1, keepdims=True)
+    dq, dk, dv, do = (DeviceBuffer.from_array(x) for x in (q, k, v, np.zeros_like(q)))
+    ops.fused_attention_ex(dq, dk, dv, do, batch=1, Tq=130, Tk=Tk, C=64, heads=1, in_dtype=MI_F32, out_dtype=MI_F32)
+    synchronize()
+    got = do.download(np.float32, q.size).reshape(q.shape)
+    assert np.abs(got - want).max() <= 2e-5 * np.sqrt(np.mean(want ** 2))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,Tq,Tk,C,heads,causal,pad,scale", [
     (1, 129, 512, 640, 10, False, 0, 0.0), (1, 300, 577, 640, 10, False, 4, 0.0), (1, 257, 700, 320, 5, True, 0, 0.0),
