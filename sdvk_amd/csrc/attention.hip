@@ -449,9 +449,11 @@ constexpr int kResidNone = 0, kResidDiagonal = 1, kResidAll = 2;
 //   * as in the fp16 kernel no row max is taken per tile: the sum of a sub-tile's P
 //     bounds each of them, and a sum over 2^8 (rare) sends the wave through a
 //     rescale;
-//   * P V = V_hi P_hi + V_lo P_hi (+ V_hi P_lo where P's residual counts, RESID as
-//     in the fp16 kernel): V_lo P_lo is below 2^-22 of a product and left out. The
-//     row sums are VALU adds, not an all-ones MFMA operand;
+//   * P V = (V_hi + V_lo) P_hi, and (V_hi + V_lo) P_lo besides where P's residual
+//     counts (RESID as in the fp16 kernel). V_lo P_lo reaches 2^-22 of a product and
+//     has one sign where V and P are near constant, so it is not left out (48.2 ->
+//     52.3 us at 1 x 10 x 2304^2). The row sums are VALU adds, not an all-ones MFMA
+//     operand;
 //   * hi = fp16(x) and lo = fp16(x - hi) take 1.5 instructions per element (packed
 //     conversion, then a mixed-precision fma that rounds straight to fp16).
 //
@@ -467,7 +469,7 @@ constexpr int kResidNone = 0, kResidDiagonal = 1, kResidAll = 2;
 // KG = 2 per CU, two waves per SIMD either way).
 //
 // What bounds it: MFMA and VALU issue, close together. Per wave, 64 keys and 32
-// queries: 24 score + 16 PV MFMAs (24 with P's residual) of 34 cycles, and 32
+// queries: 24 score + 16 PV MFMAs (32 with P's residual) of 34 cycles, and 32
 // fmas, 32 exponentials (8.5 cycles each), 32 packed conversions and 32 or 64
 // mixed fmas (9 cycles each) on the VALU. Measured on MI355X against the unpipelined
 // kernel it replaces, us: mi_fused_attention 1 x 10 x 2304^2 77.3 -> 48.7 (280
@@ -717,10 +719,12 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
         }
         if constexpr (kRes) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                o[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh[i >> 1][i & 1], frag(pl, i >> 1), o[i & 1], 0, 0, 0);
-                if (i < 2) store_unit(wst, unit0 + 2 + i);
-                if (i >= 2) read_k(kst, kt, i - 2);
+            for (int i = 0; i < 8; ++i) {
+                const int sp = i >> 2, u = i & 1;
+                const half8 v = i & 2 ? vl[sp][u] : vh[sp][u];
+                o[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v, frag(pl, sp), o[u], 0, 0, 0);
+                if (i == 0 || i == 2) store_unit(wst, unit0 + 2 + i / 2);
+                if (i == 5 || i == 7) read_k(kst, kt, i >> 2 & i >> 1 & 1);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }

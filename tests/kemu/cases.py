@@ -268,6 +268,39 @@ def attention(E, *, batch=1, Tq, Tk, C, heads, causal=False, f16_in=False, f16_o
     return assert_parity(got, want, tol=tol, what="attention")
 
 
+def residual_inputs(rng, Tq, Tk):
+    """(q, k, v) of one 64-column head whose products all have residuals of one sign:
+    P = 0.5 + p and V = 1 + v, p and v just under half an fp16 step (key 0: P = 1, V = 0)."""
+    q, k = np.zeros((Tq, 64), np.float32), np.zeros((Tk, 64), np.float32)
+    q[:, 0] = 8.0 * (1.0 - rng.uniform(0.0, 2.0 ** -16, Tq))
+    k[1:, 0] = np.log(0.5 + 2.0 ** -12 * rng.uniform(0.75, 0.95, Tk - 1))
+    v = (1.0 + 2.0 ** -11 * rng.uniform(0.75, 0.95, (Tk, 64))).astype(np.float32)
+    v[0] = 0.0
+    return q, k, v
+
+
+def residual_bias(got, q, k, v):
+    """Mean relative error against 64 bits."""
+    s = q.astype(np.float64) @ k.astype(np.float64).T / 8.0
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = p @ v.astype(np.float64) / p.sum(-1, keepdims=True)
+    return float(np.mean((got - want) / want))
+
+
+def attention_residuals(E, *, Tk, order=0, tol=2.0 ** -23):
+    """Full-precision fp32 attention on residual_inputs: a left-out product of the residuals
+    would shift every output by 0.56 to 0.9 x 2^-22; roundings are of either sign."""
+    E.order(order)
+    q, k, v = residual_inputs(np.random.default_rng(Tk), 128, Tk)
+    dq, dk, dv, do = E.buf(q), E.buf(k), E.buf(v), E.buf(np.zeros_like(q))
+    E.call("mi_fused_attention_ex", ctypes.byref(MiAttnArgs(
+        q=dq.ptr, k=dk.ptr, v=dv.ptr, out=do.ptr, batch=1, Tq=128, Tk=Tk, C=64, heads=1, causal=0, in_dtype=MI_F32,
+        out_dtype=MI_F32)), None)
+    e = abs(residual_bias(do.get(np.float32, q.size).reshape(q.shape).astype(np.float64), q, k, v))
+    assert e <= tol, f"attention_residuals: mean error {e:.2e} > {tol:.2e}"
+    return e
+
+
 # ---- full-size shapes with sampled workgroups ----------------------------------
 # The benchmark's shapes at their real size, with only a few workgroups
 # emulated (kemu_set_sample): the first one and the one that takes the last
@@ -756,7 +789,7 @@ def gguf_upload(E, *, big_rows=10240, big_cols=1280, order=0, front=False):
 
 
 CASES = {"gemm_nt": gemm_nt, "gemm_geglu": gemm_geglu, "gemm_f16a": gemm_f16a, "gemm_f16o": gemm_f16o, "gemm_nn": gemm_nn,
-         "attention": attention, "block": block,
+         "attention": attention, "attention_residuals": attention_residuals, "block": block,
          "gguf_upload": gguf_upload, "q8": q8, "glue": glue, "gemm_full": gemm_full, "gemm_nn_full": gemm_nn_full,
          "attention_full": attention_full, "block_full": block_full, "routing": routing}
 

@@ -14,11 +14,12 @@ cases: 2e-3 x RMS, the common bar).
 from __future__ import annotations
 
 import json
+import sys
 
 import numpy as np
 import pytest
 
-from test_kemu import BOTH, _run, emulator  # noqa: F401  (fixture)
+from test_kemu import BOTH, KEMU, _run, emulator  # noqa: F401  (fixture)
 
 EMULATED = [
     # two key groups: odd and even trip counts, a last tile / sub-tile of one key, a trip past the keys
@@ -79,6 +80,30 @@ def test_low_first_keys_on_gpu(gpu, oracle, Tk, n, d):
     synchronize()
     got = do.download(np.float32, q.size).reshape(q.shape)
     assert np.abs(got - want).max() <= 2e-5 * np.sqrt(np.mean(want ** 2))
+
+
+@pytest.mark.parametrize("Tk", [2, 3, 8])
+def test_no_product_of_residuals_left_out_on_emulator(emulator, Tk):  # noqa: F811
+    r = _run(dict(case="attention_residuals", Tk=Tk, schedules=BOTH))
+    assert r.returncode == 0 and r.stdout.count("OK ") == len(BOTH), (r.stdout + r.stderr)[-800:]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Tk", [2, 3])
+def test_no_product_of_residuals_left_out_on_gpu(gpu, Tk):
+    """A few keys: over many the MFMA's own accumulation has a bias of this size."""
+    sys.path.insert(0, str(KEMU))
+    from cases import residual_bias, residual_inputs
+    from sdvk_amd import MI_F32, ops
+    from sdvk_amd.hip import DeviceBuffer, synchronize
+
+    q, k, v = residual_inputs(np.random.default_rng(Tk), 128, Tk)
+    dq, dk, dv, do = (DeviceBuffer.from_array(x) for x in (q, k, v, np.zeros_like(q)))
+    ops.fused_attention_ex(dq, dk, dv, do, batch=1, Tq=128, Tk=Tk, C=64, heads=1, in_dtype=MI_F32, out_dtype=MI_F32)
+    synchronize()
+    e = residual_bias(do.download(np.float32, q.size).reshape(q.shape).astype(np.float64), q, k, v)
+    print(f"[case] {Tk} keys: mean error {e:.2e}", flush=True)
+    assert abs(e) <= 2.0 ** -23
 
 
 @pytest.mark.gpu
