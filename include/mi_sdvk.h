@@ -138,8 +138,9 @@ int mi_q8_0_quantize(const float* w, void* blocks, uint64_t n, void* stream);
  * bit. The entries without a workspace never split K across workgroups, and
  * every such call gives the same bits whatever tile build runs it (calls of up
  * to 16 rows, with or without a workspace, sum K in eight interleaved parts
- * inside a workgroup: the same bits in every entry, another grouping than the
- * tiles'). The *_ws entries may split
+ * inside a workgroup where K is a multiple of 32, the weight is below 2 GiB and
+ * no tile build is pinned by gemm_cfg: the same bits in every entry, weight
+ * layout and alignment, another grouping than the tiles'). The *_ws entries may split
  * K into the caller's workspace (partials summed in split order by a second
  * kernel): bit-identical from run to run, but grouped differently from the
  * unsplit sum (last-bit differences from the entry without a workspace).

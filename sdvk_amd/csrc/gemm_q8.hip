@@ -1410,7 +1410,7 @@ void dispatch(const GemmArgs& a, uint32_t batch, const Plan& p, float* ws, hipSt
 // The reference's scalar gemm_nt_q8 accepts any K and any row stride
 // (gemm_nt_q8.comp:52-80 stages element by element with bounds checks). Shapes
 // the tiled kernels do not take (K % 4 != 0, lda or sA not a multiple of 4, A
-// not 16-byte aligned) run here: 64 x 64 tiles, four waves of one 32 x 32 MFMA
+// not 16-byte aligned; more than kFewRows rows, or K % 32 != 0) run here: 64 x 64 tiles, four waves of one 32 x 32 MFMA
 // tile, 32 k per step, every element staged with its own bounds check
 // (zero past K). The arithmetic is the tiled kernels': A rounded to fp16, the
 // weight fp16(q * s), fp32 MFMA sums.
@@ -1559,8 +1559,10 @@ int gemm_split(const char* fn, const float* A, const uint32_t* payload, const fl
                uint32_t batch, uint64_t sA, uint64_t sC, void* ws, uint64_t ws_bytes, hipStream_t stream) {
     if (M == 0 || N == 0) return MI_OK;
     const uint32_t lda_e = lda ? lda : K;
-    // the tiled kernels stage A 16 bytes at a time; other shapes take the any-K kernel
-    const bool tiled = K % 4 == 0 && lda_e % 4 == 0 && sA % 4 == 0 && aligned(A, 16);
+    // the tiled kernels stage A 16 bytes at a time; other shapes take the any-K kernel. The
+    // few-rows kernel's A loads need the 4 bytes of every call, and it takes them all: another
+    // order of the sum for some alignments would give one product two results.
+    const bool tiled = (K % 4 == 0 && lda_e % 4 == 0 && sA % 4 == 0 && aligned(A, 16)) || few_rows(M, N, K);
     int st = validate(fn, A, payload, C, M, N, K, mode, lda, ldc, batch, sA, sC, false);
     if (st) return st;
     if (!scales) return fail(MI_ERR_INVALID_ARG, "%s: null scales", fn);

@@ -122,6 +122,28 @@ def gemm_nt(E, *, M, N, K, layout="q8_0", cfg=None, mode=0, bias=True, batch=1, 
     return assert_parity(got[mask], want[mask], tol=tol, what="gemm_nt")
 
 
+def gemm_rows_bits(E, *, M, N, K, a_off=0, pad=0, batch=1, order=0):
+    """The entries that must agree bit for bit, on one product of few rows: 34-byte
+    blocks with every operand aligned, one batch item at a time, against the split
+    layout with an A that is only 4-byte aligned (a_off floats, rows pad floats apart) in one batch."""
+    E.order(order)
+    lda, sA = K + pad, M * (K + pad) + (1 if pad else 0)
+    A, blocks = ob.normal(1, (batch - 1) * sA + M * lda), q8_weights(ob, 2, N, K)
+    payload, scales = ob.q8_0_to_split(blocks, N * K)
+    dA = E.buf(np.concatenate([np.zeros(a_off, np.float32), A]))
+    dW, dP, dS = E.buf(blocks), E.buf(payload), E.buf(scales)
+    dC = E.buf(np.zeros(batch * M * N, np.float32))
+    E.call("mi_gemm_nt_q8_split", dA.ptr + 4 * a_off, dP.ptr, dS.ptr, None, dC.ptr, M, N, K, 0, lda, 0, batch, sA, M * N,
+           None)
+    for z in range(batch):
+        rows = np.stack([A[z * sA + m * lda:z * sA + m * lda + K] for m in range(M)])
+        dR, dO = E.buf(rows), E.buf(np.zeros(M * N, np.float32))
+        E.call("mi_gemm_nt_q8_0", dR.ptr, dW.ptr, None, dO.ptr, M, N, K, 0, 0, 0, 1, 0, 0, None)
+        got, want = dC.get(np.float32)[z * M * N:(z + 1) * M * N], dO.get(np.float32)
+        assert np.array_equal(got, want), f"batch item {z}: {np.count_nonzero(got != want)} of {M * N} values differ"
+    return 0.0
+
+
 def gemm_geglu(E, *, M, F, K, cfg=None, bias=True, lda=0, ldg=0, seed=1, front=False, order=0, tol=2e-3):
     """mi_gemm_nt_q8_0_geglu: against the separate path on the same build
     (mi_gemm_nt_q8_0 into [M, 2F], then mi_geglu) to fp32 rounding, and
@@ -788,7 +810,7 @@ def gguf_upload(E, *, big_rows=10240, big_cols=1280, order=0, front=False):
     return 0.0
 
 
-CASES = {"gemm_nt": gemm_nt, "gemm_geglu": gemm_geglu, "gemm_f16a": gemm_f16a, "gemm_f16o": gemm_f16o, "gemm_nn": gemm_nn,
+CASES = {"gemm_nt": gemm_nt, "gemm_rows_bits": gemm_rows_bits, "gemm_geglu": gemm_geglu, "gemm_f16a": gemm_f16a, "gemm_f16o": gemm_f16o, "gemm_nn": gemm_nn,
          "attention": attention, "attention_residuals": attention_residuals, "block": block,
          "gguf_upload": gguf_upload, "q8": q8, "glue": glue, "gemm_full": gemm_full, "gemm_nn_full": gemm_nn_full,
          "attention_full": attention_full, "block_full": block_full, "routing": routing}
