@@ -1230,6 +1230,21 @@ void launch_cfg(const GemmArgs& a0, uint32_t batch, uint32_t splits, float* ws, 
     }
 }
 
+// k per step of the 64x64 builds in `splits` K parts: whole blocks, 128 k where K allows
+// and the longest part gains by it: a 128-k step takes as long as 1.8 to 1.9 of 64 k (MI355X).
+// K = 1280 unsplit is 10 steps of 128; in 4 parts it is 5 of 64 rather than 3 of 128
+// (154x1280x1280 8.8 vs 8.9 us, 231x1280x1280 in 3 parts 10.0 vs 10.6, 77x1280x2816 10.4 vs 10.7).
+uint32_t k_step64(uint32_t K, uint32_t splits) {
+    if (K % 128 != 0) return K % 64 != 0 ? 32 : 64;
+    return 15 * ceil_div(K / 128, splits) <= 8 * ceil_div(K / 64, splits) ? 128 : 64;
+}
+
+// The parts that launch_cfg makes of K when `splits` are asked for: whole steps, none empty.
+uint32_t launched_splits(uint32_t K, uint32_t k_step, uint32_t splits) {
+    const uint32_t steps = ceil_div(K, k_step);
+    return ceil_div(steps, ceil_div(steps, splits));
+}
+
 template <int WK, int EPI = kEpiPlain, bool AH = false>
 void launch(int cfg, const GemmArgs& a, uint32_t batch, uint32_t splits, float* ws, hipStream_t s) {
     switch (cfg) {
@@ -1267,7 +1282,7 @@ void launch(int cfg, const GemmArgs& a, uint32_t batch, uint32_t splits, float* 
                 launch_cfg<256, 256, 4, 2, 2, WK, false, 1, EPI, true, AH>(a, batch, splits, ws, s);
             break;
         default:
-            if (a.K % 128 == 0) launch_cfg<64, 64, 2, 2, 4, WK, false, 2, EPI, true, AH>(a, batch, splits, ws, s);
+            if (k_step64(a.K, splits) == 128) launch_cfg<64, 64, 2, 2, 4, WK, false, 2, EPI, true, AH>(a, batch, splits, ws, s);
             else launch_cfg<64, 64, 2, 2, 2, WK, false, 2, EPI, true, AH>(a, batch, splits, ws, s);
             break;
     }
@@ -1308,14 +1323,18 @@ struct Plan {
 //     of 256x128) 49.5 against 61.8 (128x128, 4 waves) and 57.7 (8 waves), 7904x640x640
 //     19.4 against 21.0 and 20.5, 8192x5120x640 90.5 against 91.7.
 // With a workspace (allow_split):
-//   * up to 128 64x64 tiles split K (powers of two, >= 128 k each) until about 256
-//     workgroups run: 154x1280x2048 (60 tiles x 4) 10.3 vs 15.6 unsplit. At 180 tiles
+//   * up to 128 64x64 tiles split K (split64) into the most of 8, 4, 3 or 2 parts of 128
+//     k and more that keep 256 workgroups: 154x1280x2048 (60 tiles x 4) 10.3 vs 15.6
+//     unsplit, 231x1280x1280 (80 x 3) 10.0 vs 10.2 in 4 parts. At 180 tiles
 //     two splits lose (576x1280x1280 14.1 vs 11.2 unsplit: the second launch and the
-//     partials cost more than half of a short K);
+//     partials cost more than half of a short K). Other counts lose to these: the
+//     reduce pass loads all partials of a unit at once for them alone (40x640x2048 in 8
+//     parts 7.7, in 11 9.2, in 16 10.2), and a count that whole steps do not reach runs
+//     as another (K = 1280 in 8 parts as 7: 77x640x1280 8.4, in 4 parts 7.5);
 //   * K >= 2560 on grids of up to 256 128x128 tiles: long_k_plan below.
 //
-// long_k_plan: the cheapest of the builds that fit one round, each with K split into
-// the most parts (>= 640 k) that still do. A 64-k step of a lone workgroup per CU takes
+// long_k_plan: the cheapest of the builds that fit one round, 128x128 and 256x128 each with
+// K split into the most parts (>= 640 k) that still do. A 64-k step of a lone workgroup per CU takes
 // 0.42 us on 64x64 tiles (0.65 with two per CU), 0.73 on 128x128 (8 waves), 1.05 on
 // 256x128, on top of 1.5 / 4 / 4 us per launch; partial planes cost their write and
 // read at 5 TB/s and a second launch (3.5 us). Measured against the unsplit tiles /
@@ -1324,6 +1343,15 @@ struct Plan {
 // 35.3 vs 52.6 / 47.7, 2048x1280x5120 in 3 of 256x128 48.8 vs 62.0 (128x128);
 // 1024x640x2560 stays on 64x64 (18.3; with fp16 A 15.4 vs 17.4 split), 4608x640x2560 on
 // 128x128 (34.0 vs 36.8 in 2 of 256x128).
+//
+// split64: the K parts of a 64x64 grid (1: none).
+uint32_t split64(uint64_t t64, uint32_t K) {
+    for (uint32_t splits : {8u, 4u, 3u, 2u})
+        if (t64 * splits <= kCUs && splits * 128 <= K && launched_splits(K, k_step64(K, splits), splits) == splits)
+            return splits;
+    return 1;
+}
+
 Plan long_k_plan(uint64_t t64, uint64_t t128, uint64_t t256, uint32_t K, uint64_t outputs) {
     const struct {
         int cfg;
@@ -1339,7 +1367,9 @@ Plan long_k_plan(uint64_t t64, uint64_t t128, uint64_t t256, uint32_t K, uint64_
     for (const auto& c : builds) {
         if (c.tiles > (c.split ? kCUs : 2 * kCUs)) continue;
         const uint32_t splits =
-            c.split ? static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(kCUs / c.tiles, K / 640))) : 1;
+            c.split ? launched_splits(K, K % 64 ? 32 : 64, static_cast<uint32_t>(std::max<uint64_t>(
+                                                               1, std::min<uint64_t>(kCUs / c.tiles, K / 640))))
+                    : 1;
         double us = c.launch_us + ceil_div(steps, splits) * c.step_us;
         if (splits > 1) us += 3.5 + static_cast<double>(splits) * static_cast<double>(outputs) * 8 / 5e6;
         if (us < best_us) {
@@ -1372,10 +1402,7 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, bool allow_split
     p.cfg = t128 > kCUs ? kC256x128 : t64 > 2 * kCUs ? kC128x128W8 : kC64x64;
     if (!allow_split || t128 > kCUs) return p;
     if (K >= 2560) return long_k_plan(t64, t128, t256, K, static_cast<uint64_t>(M) * N * batch);
-    if (p.cfg == kC64x64 && t64 <= kCUs / 2) {
-        const uint64_t want = (kCUs + t64 - 1) / t64;
-        while (p.splits * 2 <= want && p.splits * 2 * 128 <= K) p.splits *= 2;
-    }
+    if (p.cfg == kC64x64) p.splits = split64(t64, K);
     return p;
 }
 

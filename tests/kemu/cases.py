@@ -652,6 +652,26 @@ def routing(E, *, table, order=0):
     return 0.0
 
 
+def split_counts(E, *, shapes, order=0):
+    """The K parts that a call launches are those its workspace is sized for (no
+    workgroup emulated): one [M, N] plane per part, and no workspace for an unsplit grid."""
+    E.order(order)
+    E.lib.mi_tuning_reset()
+    E.sample("*|-|-|-")
+    bad = []
+    for M, N, K in shapes:
+        A, W, C = E.buf(nbytes=M * K * 4), E.buf(nbytes=N * K // 32 * 34), E.buf(nbytes=M * N * 4)
+        n = E.lib.mi_gemm_nt_q8_workspace_bytes(M, N, K, 1)
+        ws = E.buf(nbytes=max(n, 16))
+        E.call("mi_gemm_nt_q8_0_ws", A.ptr, W.ptr, None, C.ptr, M, N, K, 0, 0, 0, 1, 0, 0, ws.ptr, n, None)
+        parts = E.last_launch()[1][1]
+        if n != (parts * M * N * 4 if parts > 1 else 0):
+            bad.append(f"{M}x{N}x{K}: {parts} parts launched, a workspace of {n / (M * N * 4):g} planes")
+    E.sample("")
+    assert not bad, "\n".join(bad)
+    return 0.0
+
+
 def block_full(E, *, fused=False, qkv_joint=False, cached=False, order=0, half=False, hattn=False):
     """The config-4 block (level 2: 2 x 1024 tokens, C 1280, 20 heads, context
     2 x 77 x 2048, FF 1280 -> 2 x 5120 -> 1280) at full size with the first and
@@ -813,7 +833,8 @@ def gguf_upload(E, *, big_rows=10240, big_cols=1280, order=0, front=False):
 CASES = {"gemm_nt": gemm_nt, "gemm_rows_bits": gemm_rows_bits, "gemm_geglu": gemm_geglu, "gemm_f16a": gemm_f16a, "gemm_f16o": gemm_f16o, "gemm_nn": gemm_nn,
          "attention": attention, "attention_residuals": attention_residuals, "block": block,
          "gguf_upload": gguf_upload, "q8": q8, "glue": glue, "gemm_full": gemm_full, "gemm_nn_full": gemm_nn_full,
-         "attention_full": attention_full, "block_full": block_full, "routing": routing}
+         "attention_full": attention_full, "block_full": block_full, "routing": routing,
+         "split_counts": split_counts}
 
 
 def main(argv):

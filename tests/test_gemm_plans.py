@@ -21,6 +21,15 @@ ROUTES = [
     ["gemm_ws", [1152, 1280, 5120], [50, 5, 1], 512], ["gemm_ws", [1024, 640, 2560], [160, 1, 1], 256],
     ["gemm_ws", [4608, 640, 2560], [180, 1, 1], 512], ["gemm_ws", [308, 640, 2048], [50, 4, 1], 256],
 ]
+# Few tiles: K parts of 64x64 in counts that whole steps reach and that the reduce pass loads at once
+FEW_TILES = [
+    ["gemm_ws", [154, 1280, 1280], [60, 4, 1], 256], ["gemm_ws", [77, 640, 1280], [20, 4, 1], 256],
+    ["gemm_ws", [77, 640, 768], [20, 4, 1], 256], ["gemm_ws", [231, 1280, 1280], [80, 3, 1], 256],
+    ["gemm_ws", [17, 640, 2048], [10, 8, 1], 256], ["gemm_ws", [308, 1280, 1280], [100, 2, 1], 256],
+]
+COUNTS = [(M, N, K) for M in (17, 77, 154, 231, 308, 512, 576, 988) for N, K in (
+    (768, 768), (768, 3072), (1280, 1280), (1280, 5120), (640, 640), (640, 2560), (1280, 320), (1280, 2816), (320, 1280),
+    (640, 96), (640, 160), (640, 2592), (1280, 11200))]
 EMULATED = [dict(M=70, N=70, K=128, cfg="3"), dict(M=65, N=130, K=384, layout="split", front=True, mode=1),
             dict(M=70, N=66, K=640, cfg="3:2"), dict(M=64, N=64, K=192, cfg="3", layout="split"),
             dict(M=200, N=140, K=192, cfg="6", layout="split", front=True), dict(case="gemm_geglu", M=70, F=40, K=384),
@@ -30,6 +39,32 @@ EMULATED = [dict(M=70, N=70, K=128, cfg="3"), dict(M=65, N=130, K=384, layout="s
 def test_plans(emulator):  # noqa: F811
     r = _run({"case": "routing", "table": ROUTES})
     assert r.returncode == 0 and "OK routing" in r.stdout, (r.stdout + r.stderr)[-2000:]
+
+
+def test_few_tiles(emulator):  # noqa: F811
+    r = _run({"case": "routing", "table": FEW_TILES})
+    assert r.returncode == 0 and "OK routing" in r.stdout, (r.stdout + r.stderr)[-2000:]
+
+
+def test_split_counts_launched_as_planned(emulator):  # noqa: F811
+    r = _run({"case": "split_counts", "shapes": COUNTS})
+    assert r.returncode == 0 and "OK split_counts" in r.stdout, (r.stdout + r.stderr)[-2000:]
+
+
+# Split builds of the plans on few tiles: 64-k steps although K % 128 == 0, 128-k steps, an odd last part
+SPLITS = [dict(M=70, N=66, K=1280), dict(M=77, N=70, K=768, mode=1), dict(M=65, N=130, K=2560, layout="split", mode=2),
+          dict(M=40, N=64, K=2816, front=True), dict(M=70, N=66, K=640, cfg="3:5"), dict(case="gemm_f16a", M=70, N=66, K=1280)]
+
+
+def test_splits_on_emulator(emulator):  # noqa: F811
+    from concurrent.futures import ThreadPoolExecutor
+
+    specs = [dict({"case": "gemm_nt"}, schedules=BOTH, **s) for s in SPLITS]
+    with ThreadPoolExecutor(8) as ex:
+        results = list(ex.map(_run, specs))
+    bad = [f"{json.dumps(s)}\n{(r.stdout + r.stderr)[-800:]}" for s, r in zip(specs, results)
+           if r.returncode != 0 or r.stdout.count("OK ") != len(BOTH)]
+    assert not bad, "\n\n".join(bad)
 
 
 def test_steps_on_emulator(emulator):  # noqa: F811
@@ -44,7 +79,8 @@ def test_steps_on_emulator(emulator):  # noqa: F811
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,split", [(576, 1280, 5120, True), (988, 1280, 5120, True), (1152, 1280, 5120, True),
+@pytest.mark.parametrize("M,N,K,split", [(154, 1280, 1280, True), (231, 1280, 1280, True),
+                                         (77, 1280, 2816, True), (17, 320, 1280, True), (576, 1280, 5120, True), (988, 1280, 5120, True), (1152, 1280, 5120, True),
                                          (1152, 1280, 1280, False), (3952, 640, 640, False), (7904, 640, 2560, False)])
 def test_planned_shapes(gpu, oracle, tune, M, N, K, split):
     from helpers import REL_RMS_TOL, err_vs_rms, q8_weights
