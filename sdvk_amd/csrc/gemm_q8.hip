@@ -1334,7 +1334,7 @@ struct Plan {
 //   * K >= 2560 on grids of up to 256 128x128 tiles: long_k_plan below.
 //
 // long_k_plan: the cheapest of the builds that fit one round, 128x128 and 256x128 each with
-// K split into the most parts (>= 640 k) that still do. A 64-k step of a lone workgroup per CU takes
+// K split into the most parts (>= 640 k) that still do, 64x64 unsplit or as split64 has it. A 64-k step of a lone workgroup per CU takes
 // 0.42 us on 64x64 tiles (0.65 with two per CU), 0.73 on 128x128 (8 waves), 1.05 on
 // 256x128, on top of 1.5 / 4 / 4 us per launch; partial planes cost their write and
 // read at 5 TB/s and a second launch (3.5 us). Measured against the unsplit tiles /
@@ -1343,6 +1343,12 @@ struct Plan {
 // 35.3 vs 52.6 / 47.7, 2048x1280x5120 in 3 of 256x128 48.8 vs 62.0 (128x128);
 // 1024x640x2560 stays on 64x64 (18.3; with fp16 A 15.4 vs 17.4 split), 4608x640x2560 on
 // 128x128 (34.0 vs 36.8 in 2 of 256x128).
+// Few tiles: 64x64 in parts takes 5 to 6 us besides its steps and planes (two launches,
+// the first load and the last store); its price says 7.4, as the other builds' prices
+// are 1 to 2 us high there. In 8 parts of 64x64 against 128x128 in 4:
+// 77x768x3072 8.4 vs 13.8, 154x640x2560 8.9 vs 12.9, 17x1280x5120 (in 8) 9.3 vs 12.7;
+// in 4, 256x640x2560 10.1 vs 13.5, 308x768x3072 12.2 vs 15.6; 256x1280x5120 stays on 128x128 in 8
+// (17.1 vs 18.1 in 3 of 64x64).
 //
 // split64: the K parts of a 64x64 grid (1: none).
 uint32_t split64(uint64_t t64, uint32_t K) {
@@ -1376,6 +1382,14 @@ Plan long_k_plan(uint64_t t64, uint64_t t128, uint64_t t256, uint32_t K, uint64_
             best_us = us;
             best = Plan{c.cfg, splits};
         }
+    }
+    const uint32_t splits = split64(t64, K);
+    if (splits > 1) {
+        const uint32_t k_step = k_step64(K, splits);
+        const double step_us = k_step == 128 ? 0.74 : k_step == 64 ? 0.416 : 0.25;
+        const double us = 7.4 + ceil_div(ceil_div(K, k_step), splits) * step_us +
+                          static_cast<double>(splits) * static_cast<double>(outputs) * 8 / 5.5e6;
+        if (us < best_us) best = Plan{kC64x64, splits};
     }
     return best;
 }

@@ -21,8 +21,14 @@ ROUTES = [
     ["gemm_ws", [1152, 1280, 5120], [50, 5, 1], 512], ["gemm_ws", [1024, 640, 2560], [160, 1, 1], 256],
     ["gemm_ws", [4608, 640, 2560], [180, 1, 1], 512], ["gemm_ws", [308, 640, 2048], [50, 4, 1], 256],
 ]
-# Few tiles: K parts of 64x64 in counts that whole steps reach and that the reduce pass loads at once
+# Few tiles: K parts of 64x64 as long as the 128x128 tiles' parts cost more, in counts that whole
+# steps reach and that the reduce pass loads at once
 FEW_TILES = [
+    ["gemm_ws", [77, 768, 3072], [24, 8, 1], 256], ["gemm_ws", [154, 768, 3072], [36, 4, 1], 256],
+    ["gemm_ws", [77, 1280, 5120], [40, 4, 1], 256], ["gemm_ws", [154, 1280, 5120], [60, 4, 1], 256],
+    ["gemm_ws", [308, 768, 3072], [60, 4, 1], 256], ["gemm_ws", [17, 1280, 5120], [20, 8, 1], 256],
+    ["gemm_ws", [154, 640, 2560], [30, 8, 1], 256], ["gemm_ws", [256, 640, 2560], [40, 4, 1], 256],
+    ["gemm_ws", [512, 640, 2560], [80, 3, 1], 256], ["gemm_ws", [256, 1280, 5120], [20, 8, 1], 512],
     ["gemm_ws", [154, 1280, 1280], [60, 4, 1], 256], ["gemm_ws", [77, 640, 1280], [20, 4, 1], 256],
     ["gemm_ws", [77, 640, 768], [20, 4, 1], 256], ["gemm_ws", [231, 1280, 1280], [80, 3, 1], 256],
     ["gemm_ws", [17, 640, 2048], [10, 8, 1], 256], ["gemm_ws", [308, 1280, 1280], [100, 2, 1], 256],
@@ -79,8 +85,8 @@ def test_steps_on_emulator(emulator):  # noqa: F811
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,split", [(154, 1280, 1280, True), (231, 1280, 1280, True),
-                                         (77, 1280, 2816, True), (17, 320, 1280, True), (576, 1280, 5120, True), (988, 1280, 5120, True), (1152, 1280, 5120, True),
+@pytest.mark.parametrize("M,N,K,split", [(77, 768, 3072, True), (154, 1280, 1280, True), (231, 1280, 1280, True),
+                                         (77, 1280, 2816, True), (17, 640, 2560, True), (576, 1280, 5120, True), (988, 1280, 5120, True), (1152, 1280, 5120, True),
                                          (1152, 1280, 1280, False), (3952, 640, 640, False), (7904, 640, 2560, False)])
 def test_planned_shapes(gpu, oracle, tune, M, N, K, split):
     from helpers import REL_RMS_TOL, err_vs_rms, q8_weights
