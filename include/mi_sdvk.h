@@ -178,8 +178,8 @@ int mi_gemm_nt_q8_0_ws(const float* A, const void* W, const float* bias, float* 
  * of MI_GEMM_NOALLOC_SCRATCH_BYTES, held until the process ends. A shape whose
  * plan needs more scratch than that returns MI_ERR_UNSUPPORTED (no shape does
  * under the built-in tile rules: a split grid is at most 256 workgroups of
- * 256 x 128, 128 x 128 or 64 x 64 tiles, so at most 32 MiB of partials). Calls on one GPU share
- * the scratch: calls that overlap on one GPU (unordered streams) race, so
+ * 256 x 128, 128 x 128 or 64 x 64 tiles, or 2048 of 64 x 64 where K is no multiple
+ * of 64, so at most 32 MiB of partials). Calls on one GPU share the scratch: calls that overlap on one GPU (unordered streams) race, so
  * order them (one stream). Calls no hipMalloc / hipFree. The scratch's device
  * address is looked up once per GPU (hipGetSymbolAddress, which may load the
  * code object there): by mi_gemm_noalloc_init, or else by the first call on

@@ -1373,8 +1373,8 @@ Plan long_k_plan(uint64_t t64, uint64_t t128, uint64_t t256, uint32_t K, uint64_
     for (const auto& c : builds) {
         if (c.tiles > (c.split ? kCUs : 2 * kCUs)) continue;
         const uint32_t splits =
-            c.split ? launched_splits(K, K % 64 ? 32 : 64, static_cast<uint32_t>(std::max<uint64_t>(
-                                                               1, std::min<uint64_t>(kCUs / c.tiles, K / 640))))
+            c.split ? launched_splits(K, 64, static_cast<uint32_t>(std::max<uint64_t>(
+                                           1, std::min<uint64_t>(kCUs / c.tiles, K / 640))))
                     : 1;
         double us = c.launch_us + ceil_div(steps, splits) * c.step_us;
         if (splits > 1) us += 3.5 + static_cast<double>(splits) * static_cast<double>(outputs) * 8 / 5e6;
@@ -1386,10 +1386,33 @@ Plan long_k_plan(uint64_t t64, uint64_t t128, uint64_t t256, uint32_t K, uint64_
     const uint32_t splits = split64(t64, K);
     if (splits > 1) {
         const uint32_t k_step = k_step64(K, splits);
-        const double step_us = k_step == 128 ? 0.74 : k_step == 64 ? 0.416 : 0.25;
-        const double us = 7.4 + ceil_div(ceil_div(K, k_step), splits) * step_us +
+        const double us = 7.4 + ceil_div(ceil_div(K, k_step), splits) * (k_step == 128 ? 0.74 : 0.416) +
                           static_cast<double>(splits) * static_cast<double>(outputs) * 8 / 5.5e6;
         if (us < best_us) best = Plan{kC64x64, splits};
+    }
+    return best;
+}
+
+// Long K that is no multiple of 64 runs on 64x64 tiles in steps of 32 k whatever the
+// plan says (launch_general), so only their K parts are priced. A step takes 0.30 us on up
+// to 256 workgroups, 0.45 on up to 512 (two per CU), 0.65 on up to 768, then in
+// proportion; a second launch 2.1, the planes 3.5 TB/s. Measured in the parts that the
+// 128x128 tiles' price chose / these, us: 988x640x2592 (160 tiles) 24.3 / 20.0 (3 parts),
+// 768x640x5152 (120) 28.0 / 25.3 (4), 1440x1280x5152 (460) 79.7 / 71.8 (unsplit).
+Plan general_k_plan(uint64_t t64, uint32_t K, uint64_t outputs) {
+    Plan best{kC64x64, 1};
+    double best_us = 1e300;
+    for (uint32_t splits : {1u, 2u, 3u, 4u, 8u}) {
+        const uint64_t wgs = t64 * splits;
+        if (splits > 1 && (wgs > 8 * kCUs || launched_splits(K, 32, splits) != splits)) continue;
+        const double step_us = wgs <= kCUs ? 0.30 : wgs <= 2 * kCUs ? 0.45 : wgs <= 3 * kCUs ? 0.65
+                               : 0.84 * std::max(1.0, static_cast<double>(wgs) / (4 * kCUs));
+        double us = ceil_div(ceil_div(K, 32), splits) * step_us;
+        if (splits > 1) us += 2.1 + static_cast<double>(splits) * static_cast<double>(outputs) * 8 / 3.5e6;
+        if (us < best_us) {
+            best_us = us;
+            best.splits = splits;
+        }
     }
     return best;
 }
@@ -1415,7 +1438,8 @@ Plan choose(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, bool allow_split
     }
     p.cfg = t128 > kCUs ? kC256x128 : t64 > 2 * kCUs ? kC128x128W8 : kC64x64;
     if (!allow_split || t128 > kCUs) return p;
-    if (K >= 2560) return long_k_plan(t64, t128, t256, K, static_cast<uint64_t>(M) * N * batch);
+    const uint64_t outputs = static_cast<uint64_t>(M) * N * batch;
+    if (K >= 2560) return K % 64 ? general_k_plan(t64, K, outputs) : long_k_plan(t64, t128, t256, K, outputs);
     if (p.cfg == kC64x64) p.splits = split64(t64, K);
     return p;
 }

@@ -33,6 +33,12 @@ FEW_TILES = [
     ["gemm_ws", [77, 640, 768], [20, 4, 1], 256], ["gemm_ws", [231, 1280, 1280], [80, 3, 1], 256],
     ["gemm_ws", [17, 640, 2048], [10, 8, 1], 256], ["gemm_ws", [308, 1280, 1280], [100, 2, 1], 256],
 ]
+# K % 64 != 0 runs on 64x64 tiles alone: parts by their count, not by the 128x128 tiles'
+GENERAL = [
+    ["gemm_ws", [988, 640, 2592], [160, 3, 1], 256], ["gemm_ws", [768, 640, 5152], [120, 4, 1], 256],
+    ["gemm_ws", [1440, 1280, 5152], [460, 1, 1], 256], ["gemm_ws", [154, 640, 2592], [30, 8, 1], 256],
+    ["gemm_ws", [154, 1280, 3104], [60, 4, 1], 256], ["gemm_ws", [768, 1280, 5152], [240, 2, 1], 256],
+]
 COUNTS = [(M, N, K) for M in (17, 77, 154, 231, 308, 512, 576, 988) for N, K in (
     (768, 768), (768, 3072), (1280, 1280), (1280, 5120), (640, 640), (640, 2560), (1280, 320), (1280, 2816), (320, 1280),
     (640, 96), (640, 160), (640, 2592), (1280, 11200))]
@@ -47,8 +53,9 @@ def test_plans(emulator):  # noqa: F811
     assert r.returncode == 0 and "OK routing" in r.stdout, (r.stdout + r.stderr)[-2000:]
 
 
-def test_few_tiles(emulator):  # noqa: F811
-    r = _run({"case": "routing", "table": FEW_TILES})
+@pytest.mark.parametrize("table", ["FEW_TILES", "GENERAL"])
+def test_split_plans(emulator, table):  # noqa: F811
+    r = _run({"case": "routing", "table": globals()[table]})
     assert r.returncode == 0 and "OK routing" in r.stdout, (r.stdout + r.stderr)[-2000:]
 
 
@@ -86,7 +93,8 @@ def test_steps_on_emulator(emulator):  # noqa: F811
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,split", [(77, 768, 3072, True), (154, 1280, 1280, True), (231, 1280, 1280, True),
-                                         (77, 1280, 2816, True), (17, 640, 2560, True), (576, 1280, 5120, True), (988, 1280, 5120, True), (1152, 1280, 5120, True),
+                                         (77, 1280, 2816, True), (17, 640, 2560, True),
+                                         (988, 640, 2592, True), (576, 1280, 5120, True), (988, 1280, 5120, True), (1152, 1280, 5120, True),
                                          (1152, 1280, 1280, False), (3952, 640, 640, False), (7904, 640, 2560, False)])
 def test_planned_shapes(gpu, oracle, tune, M, N, K, split):
     from helpers import REL_RMS_TOL, err_vs_rms, q8_weights
