@@ -364,14 +364,28 @@ uint32_t nn_splits(uint32_t M, uint32_t N, uint32_t K, uint32_t batch) {
 // Whether the tiled kernel hands its tiles out by XCD. Workgroup i of a launch runs on
 // XCD i % 8, so with a multiple of four column tiles a column of B (all its row tiles
 // and K splits) stays on one or two XCDs by itself; with any other number the row
-// tiles that read the same B sit on up to eight, and each of their L2s fetches it. Below
-// 2 MB (half an XCD's L2) every L2 keeps all of B in either order. Measured on MI355X,
-// us, grid order / by XCD: 640x1600x5760 (7 column tiles) 45.7 / 31.5, 640x2304x5760 (9)
-// 55.1 / 43.6, 640x3456x5760 (14) 68.4 / 63.3, 1280x576x11520 (3) 48.9 / 42.1,
-// 1280x256x11520 (1) 33.3 / 27.8; the other way round 1280x1024x11520 (4) 63.8 / 65.5,
-// 640x4096x320 (16) 12.0 / 12.2, 1280x576x640 (3, 1.5 MB) 14.8 / 15.0.
-bool nn_by_xcd(uint32_t N, uint32_t K) {
-    return ceil_div(N, kBN2) % 4 != 0 && static_cast<uint64_t>(K) * N * 4 > (2u << 20);
+// tiles that read the same B sit on up to eight, and each of their L2s fetches it. By
+// XCD one L2 serves all of them instead, at its own rate. That pays (us, grid order / by
+// XCD, MI355X, another B on each call)
+//   * where the L2s' fetches take longer than one L2's service: what B (in whole tiles)
+//     exceeds an L2 by, 3.4 MB, times the row tiles (up to eight L2s), is 35 MB or more:
+//     640x1600x5760 (7 column tiles) 44.9 / 30.8, 640x2304x5760 (9) 54.8 / 37.8, 640x3456x5760
+//     (14) 62.3 / 51.6, 1280x576x11520 (3) 49.0 / 41.8, 1280x256x11520 (1) 33.6 / 28.8,
+//     1280x400x5760 (2) 27.1 / 26.0, 1280x276x6464 (2) 29.1 / 26.8;
+//   * unsplit, and on up to 72 workgroups (nine to an XCD), for a B of 2 MB and more (below,
+//     every L2 keeps all of it): 1280x4196x384 18.1 / 16.5, 640x8804x192 14.0 / 12.5,
+//     640x768x960 (45 workgroups) 16.4 / 15.8, 640x256x2880 (45) 17.3 / 16.7.
+// In between the grid's order is faster: 640x2304x640 (5.6 MB, 90 workgroups) 17.3 / 19.6, 1280x400x2560
+// (3.9) 19.2 / 22.5, 1280x576x1280 (2.8) 17.5 / 20.3, 1280x768x1920 (5.6) 21.4 / 23.0,
+// 320x2816x960 (10.3) 17.2 / 19.0, 1280x256x5760 (5.6) 23.2 / 24.0; and with a multiple of
+// four columns: 1280x1024x11520 63.8 / 65.5, 640x4096x320 12.0 / 12.2. Over 712 shapes this
+// rule is 0.2% off the faster order, the 2 MB alone 1.7%, the grid's order 6.5%.
+bool nn_by_xcd(uint32_t M, uint32_t N, uint32_t K, uint32_t batch, uint32_t splits) {
+    const uint32_t rows = ceil_div(M, kBM2), cols = ceil_div(N, kBN2);
+    const double mb = static_cast<double>(K) * batch * 4 / (1 << 20);  // of B, a column
+    if (cols % 4 == 0 || mb * N <= 2.0) return false;
+    if (rows > 1 && (splits == 1 || static_cast<uint64_t>(rows) * cols * batch * splits <= 72)) return true;
+    return (mb * cols * kBN2 - 3.4) * std::min(rows, 8u) >= 35.0;
 }
 
 int gemm_nn(const char* fn, const uint32_t* payload, const float* scales, const float* B, float* C, uint32_t M,
@@ -439,11 +453,11 @@ int gemm_nn(const char* fn, const uint32_t* payload, const float* scales, const 
         gemm_nn_q8_kernel<<<grid, 256, 0, st>>>(a);
         return check_launch(fn);
     }
-    a.by_xcd = nn_by_xcd(N, K) ? 1u : 0u;
     const uint32_t ksteps = K / kBK2;
     uint32_t splits = ws ? nn_splits(M, N, K, batch) : 1;
     const uint64_t plane = static_cast<uint64_t>(M) * N;
     if (splits > 1 && static_cast<uint64_t>(batch) * splits * plane * 4 > ws_bytes) splits = 1;
+    a.by_xcd = nn_by_xcd(M, N, K, batch, splits) ? 1u : 0u;
     if (splits > 1) {
         // partial planes into the workspace, then their sum in split order
         NnArgs p = a;

@@ -44,3 +44,15 @@ def test_bits_of_the_grid_order(gpu, oracle, tune, M, N, K, batch, mode):
         got, want = call(N, splits), call(wide, splits)
         assert np.array_equal(got[:, :, :N], want[:, :, :N])
         assert np.array_equal(got[:, :, N:], C0.reshape(batch, M, wide)[:, :, N:])
+
+
+# Both sides of the rule's edges: unsplit and split, 72 workgroups and more, one row tile, B below and
+# above what sends the row tiles to one L2
+EDGES = [(320, 2304, 640, 1), (640, 1600, 640, 2), (1280, 400, 2560, 1), (1280, 276, 6464, 1), (100, 1300, 4480, 1),
+         (256, 2308, 320, 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,batch", EDGES)
+def test_bits_at_the_edges_of_the_rule(gpu, oracle, tune, M, N, K, batch):
+    test_bits_of_the_grid_order(gpu, oracle, tune, M, N, K, batch, 0)
