@@ -538,12 +538,13 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
     float neg1 = -1.0f;
     asm volatile("" : "+v"(neg1));
     floatx4 kraw[4], vraw[4];
-    // rows past the keys read as zeros (the resource ends at key L - 1)
+    // rows past the workgroup's keys read as zeros, without a memory access (the resource ends at
+    // key kend - 1)
     auto load_k = [&](uint32_t trip) {
         const uint32_t kv0 = (trip * KG + grp) * kBKV;
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(Kp + static_cast<uint64_t>(min(kv0, L)) * a.ldk), 0,
-            static_cast<int>(tile_bytes(kv0, L, a.ldk, a.hd, 4)), 0x00020000);
+            const_cast<float*>(Kp + static_cast<uint64_t>(min(kv0, kend)) * a.ldk), 0,
+            static_cast<int>(tile_bytes(kv0, kend, a.ldk, a.hd, 4)), 0x00020000);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             kraw[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, k_off + i * 16u * k_ld4, 0, 0));
@@ -551,8 +552,8 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
     auto load_v = [&](uint32_t trip) {
         const uint32_t kv0 = (trip * KG + grp) * kBKV;
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(Vp + static_cast<uint64_t>(min(kv0, L)) * a.ldv), 0,
-            static_cast<int>(tile_bytes(kv0, L, a.ldv, a.hd, 4)), 0x00020000);
+            const_cast<float*>(Vp + static_cast<uint64_t>(min(kv0, kend)) * a.ldv), 0,
+            static_cast<int>(tile_bytes(kv0, kend, a.ldv, a.hd, 4)), 0x00020000);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             vraw[i] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, v_off + i * v_ld4, 0, 0));
@@ -769,13 +770,13 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
                 }
 #pragma unroll
             for (int i = 0; i < 8; ++i) store_unit(0, i);
-            load_k(min(1u, n - 1));
+            load_k(1u);
         }
         __syncthreads();  // every wave has read its Q rows out of the second stage
 #pragma unroll
         for (int i = 0; i < 4; ++i) store_unit(1, i);
-        load_v(min(1u, n - 1));  // V before K, as in the loop (loads retire in issue order)
-        load_k(min(2u, n - 1));
+        load_v(1u);  // V before K, as in the loop (loads retire in issue order)
+        load_k(2u);
         floatx16 s0, s1;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s0[r] = 0.0f;
@@ -793,7 +794,7 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
         // At the top of trip j: K tiles j and j + 1 and V tile j staged (or being
         // stored, before the first barrier), K tile j + 2 and V tile j + 1 on their
         // way into registers; s0 holds the scores of sub-tile 0. Past the last tile
-        // the loads repeat it: scores nobody reads.
+        // they are zeros: scores nobody reads.
         for (uint32_t j = 0; j < n; ++j) {
             const int st = j & 1;
             const uint32_t kv0 = (j * KG + grp) * kBKV;
@@ -805,14 +806,15 @@ __global__ __launch_bounds__(256 * KG, 2) void attn_f32_kernel(AttnArgs a, uint3
             __syncthreads();
             __builtin_amdgcn_sched_barrier(0);
             phase_b(std::false_type{}, st, 0, st ^ 1, 4, st ^ 1, 0);
-            load_v(min(j + 2, n - 1));
+            if (kv0 + 32 >= kend) break;  // the last trip, its second sub-tile past the keys
+            load_v(j + 2);
             __builtin_amdgcn_sched_barrier(0);
             phase_a(s1, s0, st ^ 1, 0, std::true_type{}, st, 1);
             settle(s1);
             if (kv0 + KG * kBKV + 32 > kfull) mask(s0, kv0 + KG * kBKV);
             __builtin_amdgcn_sched_barrier(0);
             phase_b(std::true_type{}, st, 1, st, 0, st ^ 1, 1);
-            load_k(min(j + 3, n - 1));
+            load_k(j + 3);
             __builtin_amdgcn_sched_barrier(0);
         }
     }

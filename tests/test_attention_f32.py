@@ -82,6 +82,33 @@ def test_low_first_keys_on_gpu(gpu, oracle, Tk, n, d):
     assert np.abs(got - want).max() <= 2e-5 * np.sqrt(np.mean(want ** 2))
 
 
+# Keys that end with a tile's first sub-tile (the loop leaves there) and one past it, in one and two
+# key groups, by the mask of a causal launch, and by the lengths of a batch
+ENDS = [dict(Tq=32, Tk=32, C=64, heads=1), dict(Tq=40, Tk=96, C=16, heads=2), dict(Tq=32, Tk=64, C=64, heads=1, causal=True),
+        dict(Tq=160, Tk=160, C=64, heads=1, causal=True), dict(Tq=20, Tk=544, C=64, heads=1), dict(Tq=20, Tk=545, C=64, heads=1),
+        dict(Tq=20, Tk=608, C=64, heads=1), dict(Tq=20, Tk=609, C=64, heads=1), dict(Tq=150, Tk=700, C=64, heads=1, causal=True),
+        dict(batch=3, Tq=9, Tk=600, C=64, heads=1, kv_len=[32, 0, 33]), dict(batch=2, Tq=9, Tk=90, C=64, heads=1, kv_len=[64, 65])]
+
+
+def test_ends_on_emulator(emulator):  # noqa: F811
+    from concurrent.futures import ThreadPoolExecutor
+
+    specs = [dict({"case": "attention"}, schedules=BOTH, precision=0, tol=2e-5, **s) for s in ENDS]
+    with ThreadPoolExecutor(8) as ex:
+        results = list(ex.map(_run, specs))
+    bad = [f"{json.dumps(s)}\n{(r.stdout + r.stderr)[-800:]}" for s, r in zip(specs, results)
+           if r.returncode != 0 or r.stdout.count("OK ") != len(BOTH)]
+    assert not bad, "\n\n".join(bad)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Tq,Tk,C,heads,causal", [
+    (1, 7, 7, 80, 5, False), (2, 26, 26, 128, 8, False), (1, 64, 64, 128, 2, True), (1, 96, 96, 64, 1, False),
+    (1, 160, 160, 640, 10, True), (1, 300, 544, 640, 10, False), (1, 300, 609, 640, 10, False)])
+def test_ends_on_gpu(gpu, oracle, B, Tq, Tk, C, heads, causal):
+    test_on_gpu(gpu, oracle, B, Tq, Tk, C, heads, causal, 0, 0.0)
+
+
 @pytest.mark.parametrize("Tk", [2, 3, 8])
 def test_no_product_of_residuals_left_out_on_emulator(emulator, Tk):  # noqa: F811
     r = _run(dict(case="attention_residuals", Tk=Tk, schedules=BOTH))
