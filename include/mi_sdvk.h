@@ -324,7 +324,8 @@ typedef struct mi_attn_args {
  * computes in fp32 throughout, fused_attn_tiled.comp:130-182). The MFMA takes
  * fp16 operands, so P = exp2(s - m) is rounded to fp16 (2^-11 relative):
  *   MI_ATTN_PREC_FP16:  one product with fp16 P (plus P's residual on the
- *                       diagonal tiles of a causal launch). Max |err| vs fp32
+ *                       diagonal tiles of a causal launch, on all of its tiles
+ *                       for fp32 inputs). Max |err| vs fp32
  *                       math up to ~2e-3 x RMS(out) on rows whose weight sits
  *                       on a few keys; typically 0.5-1.2e-3.
  *   MI_ATTN_PREC_SPLIT: P as fp16 hi + lo (lo = fp16(P - hi)) in two

@@ -472,10 +472,10 @@ constexpr int kResidNone = 0, kResidDiagonal = 1, kResidAll = 2;
 // queries: 24 score + 16 PV MFMAs (32 with P's residual) of 34 cycles, and 32
 // fmas, 32 exponentials (8.5 cycles each), 32 packed conversions and 32 or 64
 // mixed fmas (9 cycles each) on the VALU. Measured on MI355X against the unpipelined
-// kernel it replaces, us: mi_fused_attention 1 x 10 x 2304^2 77.3 -> 48.7 (280
-// TFLOP/s), 1 x 10 x 4096^2 219 -> 165, 2 x 10 x 4096^2 with fp16 P 290 -> 234, cross
-// 2 x 10 x 4096 x 77 22.8 -> 20.0; error against 64 bits 6.8e-7 -> 4.7e-7 of the
-// result's norm (2304 keys, N(0, 1) data).
+// kernel it replaces, us: mi_fused_attention 1 x 10 x 2304^2 77.0 -> 52.1 (261
+// TFLOP/s of the algorithm's operations), 1 x 10 x 4096^2 213 -> 171, 2 x 10 x 4096^2
+// with fp16 P 278 -> 226, cross 2 x 10 x 4096 x 77 22.2 -> 17.4; error against 64 bits
+// 6.8e-7 -> 4.5e-7 of the result's norm (2304 keys, N(0, 1) data).
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 // Two values as fp16 (RNE) in one packed conversion.
 __device__ __forceinline__ half2 pack2(float x, float y) { return __builtin_convertvector(floatx2{x, y}, half2); }
@@ -1552,10 +1552,10 @@ void launch_f16(const AttnArgs& a, uint32_t batch, hipStream_t s) {
 // leave no more than one on each: a grid of W workgroups with (W - 1) mod 2 CUs
 // below the CU count, and at least 512 keys, below which the second group's
 // start and the final addition cost more than it saves. Measured on MI355X, us,
-// two groups / one: 1 x 10 x 2304^2 (180 workgroups) 52.5 / 58.8, 1 x 20 x 1024^2
-// (160) 25.9 / 29.2, 2 x 10 x 4096^2 (640) 274 / 282; the other way round 2 x 20 x
-// 1024^2 (320) 52.7 / 46.8, 2 x 10 x 2304^2 (360) 104 / 99, 1 x 20 x 1024 x 77 9.5 /
-// 8.8. A causal launch carries P's residual on every tile.
+// two groups / one: 1 x 10 x 2304^2 (180 workgroups) 51.6 / 62.0, 1 x 20 x 1024^2
+// (160) 26.3 / 30.4, 2 x 10 x 4096^2 (640) 287 / 296; the other way round 2 x 20 x
+// 1024^2 (320) 53.9 / 48.1, 2 x 10 x 2304^2 (360) 108 / 103, 1 x 20 x 1024 x 77 9.1 /
+// 7.9. A causal launch carries P's residual on every tile.
 template <typename TO>
 void launch_f32(const AttnArgs& a, uint32_t batch, hipStream_t s) {
     const uint32_t qtiles = ceil_div(a.Tq, kBQ);

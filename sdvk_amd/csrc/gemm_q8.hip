@@ -517,9 +517,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_q8_kernel(GemmArgs a) {
     // and funnel-shift by 16 bits.
     uint32_t w_sh[PF][W_IT];
     // Whole-block staging: the 36-byte window at the block's 4-byte-aligned
-    // start; the row stride is 0 mod 4 (K % 64 == 0) and a step advances 34 KB
+    // start; the row stride is 0 mod 4 (K % 64 == 0) and a step advances 34 * KB
     // bytes (0 mod 4), so a block's position inside its window (0 or 2 bytes) is
-    // fixed for the lane. (Split layout: the block's 32 bytes and its scale.) v_perm selectors pick d and the eight q dwords for either.
+    // fixed for the lane. v_perm selectors pick d and the eight q dwords for either.
+    // (Split layout: the block's 32 bytes and its scale.)
     // Threads past the step's W_BLOCKS blocks still issue the loads (out of
     // range: zeros, no memory access) and store nothing: a load under a branch
     // makes the compiler's wait counts assume it was skipped, so every later
@@ -1253,6 +1254,7 @@ void launch(int cfg, const GemmArgs& a, uint32_t batch, uint32_t splits, float* 
             // three K splits 50.7 vs 53.6 (one-barrier loop; fp16 A 3-4% faster)
             launch_cfg<256, 128, 4, 2, 2, WK, false, 2, EPI, true, AH, true>(a, batch, splits, ws, s);
             break;
+        // kC128x128, kC128x64 and kC256x256: picked by no rule, pinned builds only
         case kC128x128:
             // one register set: the loop then issues most of a step's MFMAs before
             // converting the next step's loads (8192x640x2560 58 vs 68 us with two

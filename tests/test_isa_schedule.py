@@ -25,7 +25,7 @@ import isa_sched
 
 CASES = {
     "gemm_q8.hip": ("gemm_q8_kernel",),
-    "attention.hip": ("attn_f16_kernel", "attn_kernel"),
+    "attention.hip": ("attn_f16_kernel", "attn_f32_kernel", "attn_kernel"),
     "gemm_nn_q8.hip": ("gemm_nn_q8_tiled_kernel",),
 }
 

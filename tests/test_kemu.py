@@ -234,17 +234,17 @@ def test_kernels_on_emulator(emulator, family):
 
 # The tile rules at the SDXL shapes of the benchmark: (op, dims, grid, work-items
 # per workgroup). GEMM (choose in gemm_q8.hip): 192x256 (8 waves) when that gives
-# >= 120 tiles and K >= 1280 (256x128, 8 waves, when both give under one round
-# and 256x128 more tiles); 128x128 (4 waves) when that gives >= 160 tiles,
-# as 8 waves of 32x64 when those are fewer than 256 and K is not split; else
-# 64x64 (4 waves). Grid = (tiles, splits, batch). With a workspace
-# ("gemm_ws"): 128x128 grids under 256 tiles with K >= 4096 run 256x128 tiles (8
-# waves) with K split into the most parts (>= 1024 k each) with tiles x parts <= 256, 64x64
-# grids under 512 tiles split K (powers of two) to about 256 workgroups with
-# >= 128 k per split. NN GEMM: 128x256 tiles (8 waves), grid (N tiles, M tiles,
-# splits); with a workspace ("nn_ws") the most K splits with tiles x splits <= 256
-# and each split keeps >= 4 steps of 64. fp16 attention: 4-wave workgroups of
-# 128 queries, 2-wave ones of 64 when Tq <= 64.
+# >= 120 tiles and K >= 1280 over more than 640 columns (256x128, 8 waves, when both give
+# under one round and 256x128 more tiles); else the smallest tile that fits one round:
+# 64x64 (4 waves, two workgroups per CU) up to 512 tiles, 128x128 as 8 waves of 32x64 up to
+# 256, else 256x128. Grid = (tiles, splits, batch). With a workspace ("gemm_ws"): 64x64
+# grids split K into the most of 8, 4, 3 or 2 parts (>= 128 k each) that keep tiles x
+# parts <= 256; from K = 2560 on the cheapest of those and of the 128x128 and 256x128
+# tiles with K split into the most parts (>= 640 k each) that keep tiles x parts <= 256.
+# NN GEMM: 128x256 tiles (8 waves), grid (N tiles, M tiles, splits); with a workspace
+# ("nn_ws") the most K splits with tiles x splits <= 256 and each split keeps >= 4 steps
+# of 64. fp16 attention: 4-wave workgroups of 128 queries, 2-wave ones of 64 when
+# Tq <= 64.
 ROUTING = [
     ["gemm", [8192, 640, 640], [160, 1, 1], 512], ["gemm", [8192, 5120, 640], [1280, 1, 1], 512],
     ["gemm", [8192, 640, 2560], [160, 1, 1], 512], ["gemm", [2048, 1280, 1280], [160, 1, 1], 512],
